@@ -263,6 +263,12 @@ int mxm_matvec(const uint8_t* blocks, const uint8_t* scales, const void* bias, i
 const char* gq_matvec_unsupported(int type, const void* w, int64_t T, int64_t K, int64_t N, int x_dtype);
 int gq_matvec(int type, const uint8_t* w, int64_t w_bytes, const void* x, int x_dtype, int64_t T, int64_t K, void* y,
               int y_dtype, int64_t N, hipStream_t st);
+bool lg_gguf_supported(int type, const void* w, const void* x, int x_dtype, int y_dtype, int64_t T, int64_t N, int64_t K);
+int lg_gguf(int type, const uint8_t* w, int64_t w_bytes, const void* x, int64_t T, int64_t K, void* y, int64_t N,
+            hipStream_t st);
+bool lg_mxfp4_supported(const void* blocks, const void* x, int x_dtype, int y_dtype, int64_t T, int64_t N, int64_t K);
+int lg_mxfp4(const uint8_t* blocks, const uint8_t* scales, const void* bias, int bias_dtype, const void* x, int64_t T,
+             void* y, int64_t N, int64_t K, hipStream_t st);
 const char* gs_unsupported(int type, int64_t K);
 int gs_matvec(int type, const uint8_t* w, int64_t w_bytes, const void* x, int x_dtype, int64_t T, int64_t K, void* y,
               int y_dtype, int64_t N, hipStream_t st);
@@ -271,9 +277,15 @@ int gs_matvec(int type, const uint8_t* w, int64_t w_bytes, const void* x, int x_
 using namespace tsa;
 
 // Up to this many tokens per call run on the super-block streaming matvec (gguf_matvec.hip,
-// one workgroup column per token); more tokens reuse each decoded unit across a chunk of
-// tokens in the row kernel above.
+// one workgroup column per token). More bf16 tokens take the matrix cores (linear_gemm.hip;
+// Q4_K 4096 x 2048, 512 tokens: 1209 us on the row kernel above, 29 us there), other types and
+// alignments reuse each decoded unit across a chunk of tokens in the row kernel.
 constexpr int64_t GQ_MATVEC_MAX_T = 8;
+// MXFP4: the linear GEMM (linear_gemm.hip) above 32 tokens, and from 9 on where the matvec's
+// grid, one workgroup per 16 rows and 8 tokens, passes 512: 5760 x 2880 at 9 / 24 / 32 tokens
+// takes 8.2 / 8.1 / 8.2 us there and 9.6 / 19.2 / 22.6 here, 1536 x 2048 at 9 / 24 (192 / 288
+// workgroups) 7.0 / 7.2 against 5.4 / 7.2, 2048 x 768 at 32 (512) 5.5 against 4.7.
+static bool mx_gemm_better(int64_t T, int64_t N) { return T > 32 || (T > 8 && (N + 15) / 16 * ((T + 7) / 8) > 512); }
 
 extern "C" int tsa_gguf_matvec(int ggml_type, const void* w, int64_t w_bytes, const void* x, int x_dtype, int64_t T,
                                int64_t K, void* y, int y_dtype, int64_t N, void* stream) {
@@ -304,6 +316,8 @@ extern "C" int tsa_gguf_matvec(int ggml_type, const void* w, int64_t w_bytes, co
         return gs_matvec(ggml_type, wb, w_bytes, x, x_dtype, T, K, y, y_dtype, N, st);
     if (T <= GQ_MATVEC_MAX_T && !*gq_matvec_unsupported(ggml_type, w, T, K, N, x_dtype))
         return gq_matvec(ggml_type, wb, w_bytes, x, x_dtype, T, K, y, y_dtype, N, st);
+    if (T > GQ_MATVEC_MAX_T && lg_gguf_supported(ggml_type, w, x, x_dtype, y_dtype, T, N, K))
+        return lg_gguf(ggml_type, wb, w_bytes, x, T, K, y, N, st);
     const bool a16 = (reinterpret_cast<uintptr_t>(w) & 15) == 0, a2 = (reinterpret_cast<uintptr_t>(w) & 1) == 0;
     const int tch = pick_tch(T, K);
     hipError_t e;
@@ -336,6 +350,8 @@ extern "C" int tsa_mxfp4_matvec(const void* blocks, const void* scales, const vo
     const uint8_t* bl = static_cast<const uint8_t*>(blocks);
     const uint8_t* sc = static_cast<const uint8_t*>(scales);
     hipStream_t st = as_stream(stream);
+    if (mx_gemm_better(T, N) && lg_mxfp4_supported(blocks, x, x_dtype, y_dtype, T, N, K))
+        return lg_mxfp4(bl, sc, bias, bias_dtype, x, T, y, N, K, st);
     // bf16 tokens, a few at a time: the matrix-core form (mx_matvec.hip)
     if (T <= 32 && mxm_supported(blocks, x, x_dtype, N, K))
         return mxm_matvec(bl, sc, bias, bias_dtype, x, T, y, y_dtype, N, K, st);

@@ -266,9 +266,15 @@ void launch_router_decode(const void* x, int xdt, int H, const void* w, int wdt,
 }
 
 }  // namespace
+
+bool lg_bf16_supported(const void* w, int w_dtype, const void* x, int x_dtype, int y_dtype, int64_t T, int64_t N, int64_t K);
+int lg_bf16(const void* w, const void* bias, int bias_dtype, const void* x, int64_t T, void* y, int64_t N, int64_t K,
+            hipStream_t st);
+
 }  // namespace tsa
 
 using namespace tsa;
+
 
 extern "C" int tsa_router_logits(const void* x, int x_dtype, int64_t T, int64_t H, const void* w, int w_dtype,
                                  const void* bias, int bias_dtype, int64_t E, void* out, int out_dtype, void* stream) {
@@ -298,6 +304,10 @@ extern "C" int tsa_router_logits(const void* x, int x_dtype, int64_t T, int64_t 
         TSA_LAUNCH_CHECK();
         return TSA_OK;
     }
+    // bf16 batches on the matrix cores (linear_gemm.hip; 128 experts x 2048, 2048 tokens: 101 us on
+    // router_logits_kernel, 9.4 us there; 5 tokens: 10.9 and 8.1 us)
+    if (lg_bf16_supported(w, w_dtype, x, x_dtype, out_dtype, T, E, H))
+        return lg_bf16(w, bias, bias_dtype, x, T, out, E, H, as_stream(stream));
     hipLaunchKernelGGL(router_logits_kernel, dim3((unsigned)((E + 3) / 4), (unsigned)((T + RT - 1) / RT)), dim3(256), 0,
                        as_stream(stream), x, x_dtype, T, (int)H, w, w_dtype, bias, bias_dtype, (int)E, out, out_dtype);
     TSA_LAUNCH_CHECK();
