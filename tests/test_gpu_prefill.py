@@ -50,6 +50,25 @@ def test_prefill_tiled_vs_oracle(H, I, E, k, T, mfma):
                       f"prefill H={H} I={I} E={E} k={k} T={T} mfma={mfma}")
 
 
+@pytest.mark.parametrize("H,I,T", [
+    (1152, 1056, 1400),  # 9 pieces, the second GEMM's last a quarter full (H 9 x 128, I 8.25 x 128)
+    (1024, 1184, 1300),  # 8 pieces, the fewest that run on into the next tile; 9.25
+    (896, 2208, 900),    # 7 pieces: restarted per tile; 17.25, a scale group of one piece before it
+])
+def test_prefill_more_tiles_than_workgroups(H, I, T):
+    """Over 256 tiles per launch, full and partial ones: workgroups take several tiles, running
+    on from one into the next (or restarting, for short rows)."""
+    E, k = 5, 3
+    rng, L, experts, pool = _pool(H, I, E, seed=H + I)
+    x_bits = synth.bf16_normal(rng, (T, H))
+    idx, w = oex.route_topk_then_softmax(synth.zipf_logits(rng, T, E), k)
+    y = ops.moe_prefill(L, pool, torch.arange(E, dtype=torch.int32, device="cuda"),
+                        torch.from_numpy(idx.astype(np.int32)).cuda(), torch.from_numpy(w).cuda(), bf16_dev(x_bits))
+    tiles = sum(-(-c // 128) for c in np.bincount(idx.reshape(-1), minlength=E)) * -(-2 * I // 256)
+    assert tiles > 256, tiles
+    assert_close_bf16(y, _ref(experts, synth.bf16_to_f32(x_bits), idx, w), f"prefill H={H} I={I} T={T}")
+
+
 def test_prefill_only_full_row_tiles():
     """Every expert gets exactly 128 or 256 rows: the tile table holds full entries only."""
     H, I, E, k, T = 512, 256, 5, 2, 384

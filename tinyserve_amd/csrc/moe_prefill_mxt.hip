@@ -70,9 +70,6 @@ constexpr int PF_COST0 = 96;  // a tile's estimated cost is PF_COST0 + rows (mea
 constexpr int PF_QREC = 208;
 constexpr int PF_QSCALE = 192;
 constexpr int PF_QCHUNKS = PF_QREC / 16;
-static_assert(PF_BM * PF_QREC <= PF_XBYTES, "a piece of fp6 records fits an activation stage");
-constexpr int PF_HS_Q = 528;  // LDS row stride (bytes) of gate_up's fp32 outputs in the fp6 form: 128 h + 16 B
-static_assert(PF_BM * PF_HS_Q <= PF_LDS, "the staged fp32 outputs fit in the stages");
 
 struct PfEntry {
     int slot, row0, rows, expert;
@@ -206,77 +203,6 @@ __device__ __forceinline__ v16f mfma_f4f6(const v8i& a, const v8i& b, const v16f
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 4, 2, 0, sa, OPB, sb);
 }
 
-// One 128-wide piece of a wave's 64-row x 64-token block on the scaled MFMA
-// v_mfma_scale_f32_32x32x64_f8f6f4 (fp4 weights as A, fp6 activation terms as B; 2 x 2
-// blocks of 32 x 32, two K-steps of 64, each a hi and a lo product). Lane (q, r) = (lane /
-// 32, lane % 32) supplies, for K-step ks, block 2 ks + q of weight row r: the 16 bytes of
-// its 16-row tile's lane 16 (2 ks + q) + r % 16 and that lane's scale byte for the piece;
-// and of token column r: the block's 24 bytes of hi (or lo) codes and its scale, which the
-// instruction takes from byte 2 ks of the scale word shifted down by q bytes. Blocks at
-// or past K get a zero weight operand with a unit scale (their activation records are
-// zero, but the weight bytes and scales there belong to the next tile).
-template <int NB>
-__device__ __forceinline__ void pf_piece_q6(v16f (&acc)[2][2], const uint8_t* xs, const uint8_t* ws,
-                                            const uint8_t* ss, int mp, int K, int wn, int wt, int lane) {
-    const int q = lane >> 5, rr = lane & 31;
-    v8i A[2][2];
-    int sa[2][2];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-        const int rt = 4 * wn + 2 * rb + (rr >> 4);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int lt = 16 * (2 * ks + q) + (rr & 15);
-            const u32x4 w = *reinterpret_cast<const u32x4*>(ws + rt * 1024 + 16 * lt);
-            A[rb][ks] = v8i{(int)w[0], (int)w[1], (int)w[2], (int)w[3], 0, 0, 0, 0};
-            sa[rb][ks] = ss[rt * 256 + 4 * lt + (mp & 3)];
-        }
-    }
-    if (128 * (mp + 1) > K) {  // the row's last, partial piece
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                if (128 * mp + 32 * (2 * ks + q) >= K) {
-                    A[rb][ks] = v8i{0, 0, 0, 0, 0, 0, 0, 0};
-                    sa[rb][ks] = 127;
-                }
-    }
-    v8i Bh[2][NB], Bl[2][NB];
-    int sh[NB], sl[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const uint8_t* rec = xs + (64 * wt + 32 * b + rr) * PF_QREC;
-        sh[b] = (int)(*reinterpret_cast<const uint32_t*>(rec + PF_QSCALE) >> (8 * q));
-        sl[b] = sh[b] - 0x05050505;  // lo scale = hi scale - 5 (every scale byte is >= 5)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const uint8_t* blk = rec + 48 * (2 * ks + q);
-            const u32x4 d0 = *reinterpret_cast<const u32x4*>(blk);
-            const u32x4 d1 = *reinterpret_cast<const u32x4*>(blk + 16);
-            const u32x4 d2 = *reinterpret_cast<const u32x4*>(blk + 32);
-            Bh[ks][b] = v8i{(int)d0[0], (int)d0[1], (int)d0[2], (int)d0[3], (int)d1[0], (int)d1[1], 0, 0};
-            Bl[ks][b] = v8i{(int)d1[2], (int)d1[3], (int)d2[0], (int)d2[1], (int)d2[2], (int)d2[3], 0, 0};
-        }
-    }
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[rb][b] = mfma_f4f6<0>(A[rb][0], Bh[0][b], acc[rb][b], sa[rb][0], sh[b]);
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[rb][b] = mfma_f4f6<0>(A[rb][0], Bl[0][b], acc[rb][b], sa[rb][0], sl[b]);
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[rb][b] = mfma_f4f6<2>(A[rb][1], Bh[1][b], acc[rb][b], sa[rb][1], sh[b]);
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[rb][b] = mfma_f4f6<2>(A[rb][1], Bl[1][b], acc[rb][b], sa[rb][1], sl[b]);
-}
-
 // The K loop of one tile, as a stream of steps s = -PF_WAHEAD .. MP - 1: step s waits for
 // and multiplies piece s (s >= 0), then issues the activations of piece s + PF_XAHEAD and
 // the weights of piece s + PF_WAHEAD, in that order. The weights of piece i therefore go
@@ -284,7 +210,7 @@ __device__ __forceinline__ void pf_piece_q6(v16f (&acc)[2][2], const uint8_t* xs
 // complete, W(s) and its scale word are too; the loads newer than X(s) are counted
 // exactly (never fewer than issued: a wait for fewer outstanding is only stricter). NB = 0:
 // the wave has no live block in this tile and only takes part in the loads and barriers.
-template <int NB, bool Q6, class IX, class IW, class WL>
+template <int NB, class IX, class IW, class WL>
 __device__ __forceinline__ void pf_kloop(v16f (&acc)[2][2], IX& issue_x, IW& issue_w, WL& w_loads, int MP, int K,
                                          int wn, int wt, int lane) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -302,13 +228,12 @@ __device__ __forceinline__ void pf_kloop(v16f (&acc)[2][2], IX& issue_x, IW& iss
             const uint8_t* xs = smem + (st % PF_XST) * PF_XBYTES;
             const uint8_t* ws = smem + PF_WOFF + (st % PF_WST) * PF_WBYTES;
             const uint8_t* ss = smem + PF_SOFF + ((st >> 2) & 1) * PF_SBYTES;
-            if constexpr (Q6) pf_piece_q6<NB ? NB : 1>(acc, xs, ws, ss, st, K, wn, wt, lane);
-            else pf_piece<NB ? NB : 1>(acc, xs, ws, ss, st, K, wn, wt, lane);
+            pf_piece<NB ? NB : 1>(acc, xs, ws, ss, st, K, wn, wt, lane);
         }
     }
 }
 
-template <bool GATE_UP, bool Q6>
+template <bool GATE_UP>
 __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
@@ -339,24 +264,13 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
         // s = lane % 16 the row's 16-byte chunk s ^ (token % 16). The swizzle keeps the B
         // fragment reads (one chunk of 32 tokens per lane group) free of bank conflicts.
         // Tokens past the tile's rows re-read token 0's row (their columns are dropped).
-        // fp6 form: the piece's 128 records are 13 x 128 chunks of 16 bytes, chunk i at LDS
-        // offset 16 i; instruction c of wave w carries chunks 64 (4 w + c) + lane (those past
-        // the tile's rows, and the 384 past 128 records, re-read token 0's and land in the
-        // unused end of the stage).
         uint32_t xoff[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            int tok, ch = 0;
-            if constexpr (Q6) {
-                const int ci = 64 * (4 * wave + c) + lane;
-                tok = ci / PF_QCHUNKS;
-                ch = ci - PF_QCHUNKS * tok;
-            } else {
-                tok = 16 * wave + 4 * c + (lane >> 4);
-            }
+            int tok = 16 * wave + 4 * c + (lane >> 4);
             if (tok >= rows) tok = 0;
             const int64_t srow = GATE_UP ? p.perm[row0 + tok] / p.k : row0 + tok;
-            xoff[c] = (uint32_t)(srow * p.src_stride + 16 * ch);
+            xoff[c] = (uint32_t)(srow * p.src_stride);
         }
         // Weight DMA: wave w fills row tiles 2w, 2w+1 of the workgroup's 16; one resource
         // spans the workgroup's live tiles (tiles past N read zero).
@@ -372,11 +286,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
         const uint32_t sb = (uint32_t)p.stile_bytes;
         auto issue_x = [&](int mp) {
             const uint32_t st = lds0 + (uint32_t)((mp % PF_XST) * PF_XBYTES) + 16 * wave * 256;
-            if constexpr (Q6) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) pf_dma(xr, xoff[c] + PF_QREC * mp, st + c * 1024);
-                return;
-            }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int tok = 16 * wave + 4 * c + (lane >> 4);
@@ -427,9 +336,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
                 for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
         // One K loop per live-subtile count, so the accumulators keep one register home
         // (a per-piece branch made the compiler copy them after every piece).
-        if (!active) pf_kloop<0, Q6>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
-        else if (nsub == 2) pf_kloop<2, Q6>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
-        else pf_kloop<1, Q6>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
+        if (!active) pf_kloop<0>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
+        else if (nsub == 2) pf_kloop<2>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
+        else pf_kloop<1>(acc, issue_x, issue_w, w_loads, MP, K, wn, wt, lane);
         if (tid == 0) s_next = grabbed;
         __syncthreads();  // every wave is done with the last stages before the next tile refills them
         tl = uniform(s_next);  // rewritten only after the next tile's K loop, which has a barrier per piece
@@ -438,7 +347,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
         // per token (the stages are free: every wave is past the K loop's last LDS read).
         // acc[rb][b][4u + r] is row 32 rb + 8u + 4g + r of the wave's 64 (r = 0..3), token
         // column 64 wt + 32 b + (lane % 32).
-        constexpr int HS = GATE_UP ? (Q6 ? PF_HS_Q : PF_HS_GU) : PF_HS_DN;
+        constexpr int HS = GATE_UP ? PF_HS_GU : PF_HS_DN;
         if (active) {
 #pragma unroll
             for (int rb = 0; rb < 2; ++rb) {
@@ -454,10 +363,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
                         const int tk = 64 * wt + 32 * b + rr;
                         if (b >= nsub || tk >= rows) continue;
                         const v4f v = v4f{acc[rb][b][4 * u], acc[rb][b][4 * u + 1], acc[rb][b][4 * u + 2], acc[rb][b][4 * u + 3]} + bias;
-                        if (GATE_UP && Q6)
-                            *reinterpret_cast<float2*>(smem + tk * HS + 2 * c) =
-                                make_float2(swiglu_oai_fast(p.L, v[0], v[1]), swiglu_oai_fast(p.L, v[2], v[3]));
-                        else if (GATE_UP)
+                        if (GATE_UP)
                             *reinterpret_cast<uint32_t*>(smem + tk * HS + c) =
                                 pack_bf16x2(swiglu_oai_fast(p.L, v[0], v[1]), swiglu_oai_fast(p.L, v[2], v[3]));
                         else
@@ -467,54 +373,533 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
             }
         }
         __syncthreads();
-        // 2, fp6 form of gate_up: thread (token tk, block bq) turns h[row0 + tk, 128 nt + 32 bq ..]
-        // into its fp6 terms, written to record nt of the row (blocks past the row's end as
-        // zero codes with a unit scale: the down GEMM multiplies them by zero weights).
-        if constexpr (GATE_UP && Q6) {
-            const int tk = tid & (PF_BM - 1), bq = tid >> 7;
-            if (tk < rows) {
-                uint32_t hi[6], lo[6], sc = 127u;
-                const int c0 = 128 * nt + 32 * bq;
-                if (c0 < N / 2) {
-                    float v[32];
+        // 2: whole rows out, 16 bytes (8 values) per lane, consecutive lanes along a row:
+        // gate_up h[row0 + tk, 128 nt ..] (256 B a row), down yk[perm[row0 + tk], 256 nt ..] (512 B).
+        constexpr int CPR = GATE_UP ? 16 : 32;  // 16-byte chunks per row
+        const int ncol = GATE_UP ? N / 2 - 128 * nt : N - 256 * nt;  // live values in the row (multiple of 8)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const v4f f = *reinterpret_cast<const v4f*>(smem + tk * HS + 128 * bq + 16 * i);
-                        v[4 * i] = f[0];
-                        v[4 * i + 1] = f[1];
-                        v[4 * i + 2] = f[2];
-                        v[4 * i + 3] = f[3];
-                    }
-                    sc = fp6_terms(v, hi, lo);
-                } else {
-#pragma unroll
-                    for (int d = 0; d < 6; ++d) hi[d] = lo[d] = 0u;
-                }
-                uint8_t* rec = p.qout + (int64_t)(row0 + tk) * p.out_stride + (int64_t)nt * PF_QREC;
-                *reinterpret_cast<uint4*>(rec + 48 * bq) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                *reinterpret_cast<uint4*>(rec + 48 * bq + 16) = make_uint4(hi[4], hi[5], lo[0], lo[1]);
-                *reinterpret_cast<uint4*>(rec + 48 * bq + 32) = make_uint4(lo[2], lo[3], lo[4], lo[5]);
-                rec[PF_QSCALE + bq] = (uint8_t)sc;
-            }
-        } else {
-            // 2: whole rows out, 16 bytes (8 values) per lane, consecutive lanes along a row:
-            // gate_up h[row0 + tk, 128 nt ..] (256 B a row), down yk[perm[row0 + tk], 256 nt ..] (512 B).
-            constexpr int CPR = GATE_UP ? 16 : 32;  // 16-byte chunks per row
-            const int ncol = GATE_UP ? N / 2 - 128 * nt : N - 256 * nt;  // live values in the row (multiple of 8)
-#pragma unroll
-            for (int j = 0; j < PF_BM * CPR / PF_THREADS; ++j) {
-                const int i = tid + PF_THREADS * j, tk = i / CPR, ch = i % CPR;
-                if (tk >= rows || 8 * ch >= ncol) continue;
-                const uint4 v = *reinterpret_cast<const uint4*>(smem + tk * HS + 16 * ch);
-                if (GATE_UP) {
-                    *reinterpret_cast<uint4*>(p.out + (int64_t)(row0 + tk) * (N / 2) + 128 * nt + 8 * ch) = v;
-                } else {
-                    const int64_t asg = p.perm[row0 + tk];
-                    *reinterpret_cast<uint4*>(p.out + asg * N + 256 * nt + 8 * ch) = v;
-                }
+        for (int j = 0; j < PF_BM * CPR / PF_THREADS; ++j) {
+            const int i = tid + PF_THREADS * j, tk = i / CPR, ch = i % CPR;
+            if (tk >= rows || 8 * ch >= ncol) continue;
+            const uint4 v = *reinterpret_cast<const uint4*>(smem + tk * HS + 16 * ch);
+            if (GATE_UP) {
+                *reinterpret_cast<uint4*>(p.out + (int64_t)(row0 + tk) * (N / 2) + 128 * nt + 8 * ch) = v;
+            } else {
+                const int64_t asg = p.perm[row0 + tk];
+                *reinterpret_cast<uint4*>(p.out + asg * N + 256 * nt + 8 * ch) = v;
             }
         }
         __syncthreads();  // the staged rows are read before the next tile's loads refill the stages
+    }
+}
+
+// ---- the fp6 form's GEMM (pf6_gemm_kernel)
+//
+// The same tile (256 weight rows x 128 sorted rows, wave (wn, wt) 64 x 64), schedule and sorted
+// rows as pf_gemm_kernel, on v_mfma_scale_f32_32x32x64_f8f6f4 with the weights as stored (fp4,
+// e8m0 scales) against the activations' fp6 hi and lo terms. What bounds it: the LDS (a piece
+// moves about 43 KB in and 132 KB out of it, as long as its 128 MFMAs take) and the copies,
+// with the matrix cores busy a third of the time; so the K loop is kept free of everything
+// else:
+//  - one stream of pieces over all of a workgroup's tiles: the next tile is asked for as a tile
+//    starts, and its first pieces are copied while the last ones multiply and the epilogue,
+//    which works in registers, runs (rows of fewer than P6_STREAM pieces restart per tile);
+//  - activations are copied by waves 0 .. 3 and weights by waves 4 .. 7, so each wave waits
+//    only for its own kind: loads return in order, and a wave waiting for the activations 2
+//    pieces ahead would also wait for the weights 3 ahead;
+//  - a K step's operands are read while the step before multiplies, across the barrier;
+//  - stage positions are running byte offsets, LDS destinations immediates of the copies; the
+//    steady part of the loop has no tail checks, the tile's last 4 pieces are written out.
+// 2880 x 2880, top-4 of 32 experts, whole call (us; one loop with all reads and waits at its top
+// before, now): 2048 tokens 453 -> 425, 700 260 -> 238, 128 162 -> 148, 24 125 -> 115, 5 83 -> 77.
+// (Reads and copies placed between the MFMAs instead of ahead of them: 436 us at 2048 tokens.)
+
+// LDS of pf6_gemm_kernel: three activation stages, four weight stages, a ring of three scale
+// groups (one word per lane of the 16 row tiles: 4 pieces), two tiles' biases and permutations.
+constexpr int P6_XB = PF_BM * PF_QREC;  // 26 KB
+constexpr int P6_XST = 3, P6_WST = 4;
+constexpr int P6_WOFF = P6_XST * P6_XB;
+constexpr int P6_SOFF = P6_WOFF + P6_WST * PF_WBYTES;
+constexpr int P6_BOFF = P6_SOFF + 3 * PF_SBYTES;
+constexpr int P6_POFF = P6_BOFF + 2 * 1024;
+constexpr int P6_LDS = P6_POFF + 2 * PF_BM * 4;
+static_assert(P6_LDS <= 160 * 1024, "LDS per workgroup");
+constexpr int P6_STREAM = 8;  // rows of at least this many pieces run on into the next tile (fewer cannot:
+                              // the next tile is known after 3 pieces, its copies start 4 before the end)
+
+// pf_dma / pf_dma4 to lds + IMM, with a scalar byte offset soff added to voff.
+template <int IMM>
+__device__ __forceinline__ void p6_dma(const v4i& r, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
+                 "s"(__builtin_amdgcn_readfirstlane((int)lds)), "n"(IMM)
+                 : "memory", "m0", "scc");
+}
+template <int IMM>
+__device__ __forceinline__ void p6_dma4(const v4i& r, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
+                 "s"(__builtin_amdgcn_readfirstlane((int)lds)), "n"(IMM)
+                 : "memory", "m0", "scc");
+}
+
+// One table entry by a scalar load (after an inline-assembly copy the compiler would use a
+// vector load, whose wait would also wait for the copies).
+__device__ __forceinline__ PfEntry p6_entry(const PfEntry* t) {
+    v4i e;
+    asm volatile("s_load_dwordx4 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(e) : "s"(t) : "memory");
+    return PfEntry{e[0], e[1], e[2], e[3]};
+}
+
+// One K step's operands (64 values: blocks 2 ks + q of a piece) of a wave's 64 rows x 64 tokens
+// on v_mfma_scale_f32_32x32x64_f8f6f4, 2 x 2 blocks of 32 x 32: lane (q, r) = (lane / 32,
+// lane % 32) holds the 16 bytes of block 2 ks + q of weight row 32 rb + r and its scale byte,
+// and that block's 24 bytes of hi and 24 of lo codes of token column 32 b + r.
+typedef uint32_t u32x12 __attribute__((ext_vector_type(12)));
+struct P6Ops {
+    u32x4 A[2];
+    u32x12 B[2];  // hi in dwords 0 .. 5, lo in 6 .. 11
+    int sa[2];
+};
+
+template <bool GATE_UP>
+__global__ void __launch_bounds__(PF_THREADS) pf6_gemm_kernel(PfGemm p) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ int s_next;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    const int wn = wave & 3, wt = wave >> 2, q = lane >> 5, rr = lane & 31;
+    const int N = p.N, K = p.K, MP = p.MP, NT = p.NT;
+    const int xcd = blockIdx.x & 7, R = gridDim.x >> 3;
+    const int m0 = uniform(p.n_entries[1 + xcd]);
+    const int total = (uniform(p.n_entries[2 + xcd]) - m0) * NT;  // this XCD's tiles
+    int* const ctr = p.ctr + PF_CTR_STRIDE * xcd;
+    const int W = (int)(p.stile_bytes >> 8);  // scale words per lane
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+    const v4i xr = buf_desc(p.src, (uint32_t)(p.src_rows * p.src_stride));
+    const uint32_t tb = (uint32_t)p.tile_bytes, sb = (uint32_t)p.stile_bytes;
+    const int bes = p.L.bias_dtype == TSA_F32 ? 4 : 2;
+    const bool xw = wave < 4;                 // waves 0 .. 3 copy activations, 4 .. 7 weights and scales
+    const bool stream = MP >= P6_STREAM;
+
+    // The first tile of workgroup b is b / 8; later ones come from the counter (offset by R,
+    // so the first R are never handed out twice).
+    int tl = (int)(blockIdx.x >> 3);
+    if (tl >= total) return;
+
+    struct Tile { int row0, rows, nt; const uint8_t* base; };
+    auto tile = [&](int t) {
+        const int m = t / NT;
+        const PfEntry e = p6_entry(p.table + m0 + m);
+        return Tile{e.row0, e.rows, t - m * NT, p.pool + (int64_t)e.slot * p.L.slot_bytes};
+    };
+
+    int xg = 0, wg = 0, sg = 0;  // byte offsets of the stage / slot the next piece is copied into
+    int xc = 0, wc = 0, sc = 0;  // ... and of the current piece's
+    auto next3 = [](int v, int step) { return v == 2 * step ? 0 : v + step; };
+    auto next4 = [](int v, int step) { return v == 3 * step ? 0 : v + step; };
+
+    // What the copying waves hold of the tile they copy. Activations: instruction i of a piece's
+    // 26 carries 16-byte chunks 64 i + lane of its 128 records (wave w: i = w + 4 c); rows past
+    // the tile re-read token 0's, and whole instructions past the last 32 rows are left out
+    // (their columns are dropped). Weights: wave 4 + w fills row tiles 4 w .. 4 w + 3.
+    uint32_t xoff[7];
+    int xin = 0;
+    v4i wr = xr, sr = xr;
+    auto copy_perm = [&](const Tile& t, int ps) {  // wave 1: the tile's 128 permutation entries
+        if (wave == 1) {
+            const v4i pr = buf_desc(p.perm + t.row0, 4u * (uint32_t)t.rows);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) pf_dma4(pr, 256 * i + 4 * lane, lds0 + P6_POFF + 512 * ps + 256 * i);
+        }
+    };
+    auto set_x = [&](const Tile& t, int ps) {
+        xin = (((t.rows + 31) & ~31) * PF_QCHUNKS + 63) / 64;
+        if (!xw) return;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // per tile, not kept in registers over the K loop
+        const uint32_t stride = (uint32_t)p.src_stride;
+#pragma unroll
+        for (int c = 0; c < 7; ++c) {
+            const uint32_t ci = 64 * (wave + 4 * c) + ln;
+            uint32_t tok = ci / PF_QCHUNKS;
+            const uint32_t ch = ci - PF_QCHUNKS * tok;
+            if ((int)tok >= t.rows) tok = 0;
+            const uint32_t srow =
+                GATE_UP ? *reinterpret_cast<const uint32_t*>(smem + P6_POFF + 512 * ps + 4 * tok) / (uint32_t)p.k : t.row0 + tok;
+            xoff[c] = srow * stride + 16 * ch;
+        }
+    };
+    auto set_w = [&](const Tile& t) {
+        const int rtw = t.nt * (PF_BN / 16);
+        int nrw = N / 16 - rtw;
+        nrw = nrw > PF_BN / 16 ? PF_BN / 16 : nrw;  // tiles past N read zero
+        wr = buf_desc(t.base + p.w_off + (int64_t)rtw * p.tile_bytes, (uint32_t)nrw * tb);
+        sr = buf_desc(t.base + p.s_off + (int64_t)rtw * p.stile_bytes, (uint32_t)nrw * sb);
+    };
+    // Piece mp of the tile set last, into its stage (the bias with the first activations).
+    auto issue_x = [&](const Tile& t, int mp, int bs) {
+        if (mp == 0 && wave == 0 && p.b_off >= 0) {
+            const int64_t brows = N - PF_BN * t.nt;
+            const v4i br = buf_desc(t.base + p.b_off + (int64_t)PF_BN * t.nt * bes, (uint32_t)(brows > 0 ? brows * bes : 0));
+            for (int i = 0; i < bes; ++i) pf_dma4(br, 256 * i + 4 * lane, lds0 + P6_BOFF + 1024 * bs + 256 * i);
+        }
+        const uint32_t dst = lds0 + (uint32_t)xg + 1024u * (uint32_t)wave, so = (uint32_t)mp * PF_QREC;
+        if (xin == 26) {  // more than 96 rows: every instruction (6 or 7 of each wave)
+            p6_dma<0>(xr, xoff[0], so, dst);
+            p6_dma<4096>(xr, xoff[1], so, dst);
+            p6_dma<2 * 4096>(xr, xoff[2], so, dst);
+            p6_dma<3 * 4096>(xr, xoff[3], so, dst);
+            p6_dma<4 * 4096>(xr, xoff[4], so, dst);
+            p6_dma<5 * 4096>(xr, xoff[5], so, dst);
+            if (wave < 2) p6_dma<6 * 4096>(xr, xoff[6], so, dst);
+        } else {
+            p6_dma<0>(xr, xoff[0], so, dst);
+            if (wave + 4 < xin) p6_dma<4096>(xr, xoff[1], so, dst);
+            if (wave + 8 < xin) p6_dma<2 * 4096>(xr, xoff[2], so, dst);
+            if (wave + 12 < xin) p6_dma<3 * 4096>(xr, xoff[3], so, dst);
+            if (wave + 16 < xin) p6_dma<4 * 4096>(xr, xoff[4], so, dst);
+        }
+    };
+    const uint32_t t4 = 4 * (uint32_t)(wave & 3);
+    uint32_t wo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wo[i] = (t4 + i) * tb + 16 * lane;
+    auto issue_w = [&](int mp) {  // 4 loads, and 4 of the group's scale words when mp % 4 == 0
+        const uint32_t dst = lds0 + P6_WOFF + (uint32_t)wg + 1024u * t4, so = 1024u * (uint32_t)mp;
+        p6_dma<0>(wr, wo[0], so, dst);
+        p6_dma<1024>(wr, wo[1], so, dst);
+        p6_dma<2048>(wr, wo[2], so, dst);
+        p6_dma<3072>(wr, wo[3], so, dst);
+        if ((mp & 3) == 0) {
+            const int w = mp >> 2, nw = W - 4 * (w >> 2) < 4 ? W - 4 * (w >> 2) : 4;
+            const uint32_t sd = lds0 + P6_SOFF + (uint32_t)sg + 256u * t4, v = t4 * sb + 4 * nw * lane;
+            const uint32_t ss = 1024 * (w >> 2) + 4 * (w & 3);
+            p6_dma4<0>(sr, v, ss, sd);
+            p6_dma4<256>(sr, v + sb, ss, sd);
+            p6_dma4<512>(sr, v + 2 * sb, ss, sd);
+            p6_dma4<768>(sr, v + 3 * sb, ss, sd);
+        }
+    };
+    // every wave keeps every position (a store behind a branch on the wave's role would put them
+    // in memory): after activations, and after weights of piece mp (end: the tile's last)
+    auto next_x = [&]() { xg = next3(xg, P6_XB); };
+    auto next_w = [&](int mp, bool end) {
+        wg = next4(wg, PF_WBYTES);
+        sg = (mp & 3) == 3 || end ? next3(sg, PF_SBYTES) : sg;
+    };
+
+    P6Ops o0, o1;
+    int sh[2];
+    uint32_t shn[2] = {0u, 0u};
+
+    // Operand reads: lane-dependent bases, everything else scalar or an immediate. Blocks at or
+    // past K get a zero weight operand with a unit scale (their activation records are zero, but
+    // the weight bytes and scales there belong to the next tile).
+    const uint8_t* const xb = smem + (64 * wt + rr) * PF_QREC + 48 * q;
+    const uint8_t* const xsb = smem + (64 * wt + rr) * PF_QREC + PF_QSCALE;
+    const uint8_t* const wb = smem + P6_WOFF + (4 * wn + (rr >> 4)) * 1024 + 16 * (16 * q + (rr & 15));
+    const uint8_t* const sbp = smem + P6_SOFF + (4 * wn + (rr >> 4)) * 256 + 4 * (16 * q + (rr & 15));
+    auto read_a = [&](P6Ops& o, int ks, int mp) {
+        const uint8_t* w = wb + wc + 512 * ks;
+        const uint8_t* s = sbp + sc + (mp & 3) + 128 * ks;
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+            o.A[rb] = *reinterpret_cast<const u32x4*>(w + 2048 * rb);
+            o.sa[rb] = s[512 * rb];
+        }
+    };
+    auto read_b = [&](P6Ops& o, int ks, int b) {
+        const u32x4* xp = reinterpret_cast<const u32x4*>(xb + xc + 96 * ks + 32 * b * PF_QREC);
+        const u32x4 d0 = xp[0], d1 = xp[1], d2 = xp[2];
+        const auto d01 = __builtin_shufflevector(d0, d1, 0, 1, 2, 3, 4, 5, 6, 7);
+        const auto d2x = __builtin_shufflevector(d2, d2, 0, 1, 2, 3, -1, -1, -1, -1);
+        o.B[b] = __builtin_shufflevector(d01, d2x, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11);
+    };
+    auto past_k = [&](P6Ops& o, int ks, int mp, bool tail) {
+        if (tail && 128 * mp + 64 * ks + 64 > K && 128 * mp + 32 * (2 * ks + q) >= K) {
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb) {
+                o.A[rb] = u32x4{0u, 0u, 0u, 0u};
+                o.sa[rb] = 127;
+            }
+        }
+    };
+    // the two columns' hi scales of a piece: block q in byte 0, block 2 + q in byte 2
+    auto read_scales = [&]() {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            shn[b] = *reinterpret_cast<const uint32_t*>(xsb + xc + 32 * b * PF_QREC);
+    };
+    auto use_scales = [&]() {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) sh[b] = (int)(shn[b] >> (8 * q));
+    };
+
+    v16f acc[2][2];
+    int nsub = 0;  // the wave's live 32-token columns
+    // One column's hi or lo products of a K step, both row blocks.
+    auto mul = [&](const P6Ops& o, auto ksc, int b, bool low) {
+        constexpr int KS = decltype(ksc)::value;
+        if (nsub <= b) return;
+        const v8i t = low ? __builtin_bit_cast(v8i, __builtin_shufflevector(o.B[b], o.B[b], 6, 7, 8, 9, 10, 11, -1, -1))
+                          : __builtin_bit_cast(v8i, __builtin_shufflevector(o.B[b], o.B[b], 0, 1, 2, 3, 4, 5, -1, -1));
+        const int sb = low ? sh[b] - 0x05050505 : sh[b];  // lo scale = hi scale - 5 (every scale byte is >= 5)
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+            acc[rb][b] = mfma_f4f6<2 * KS>(
+                __builtin_bit_cast(v8i, __builtin_shufflevector(o.A[rb], o.A[rb], 0, 1, 2, 3, -1, -1, -1, -1)), t, acc[rb][b],
+                o.sa[rb], sb);
+    };
+    // the MFMAs stay on this side of the next barrier (the compiler would sink them past it)
+    auto pin = [&]() {
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) asm volatile("" : "+v"(acc[rb][b]));
+    };
+    // Step 1's operands are read while step 0 multiplies ..
+    using K0 = std::integral_constant<int, 0>;
+    using K1 = std::integral_constant<int, 1>;
+    auto front = [&](int mp, bool tail) {
+        read_a(o1, 1, mp);
+        read_b(o1, 1, 0);
+        read_b(o1, 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(o0, K0{}, 0, false);
+        mul(o0, K0{}, 0, true);
+        mul(o0, K0{}, 1, false);
+        mul(o0, K0{}, 1, true);
+        __builtin_amdgcn_sched_barrier(0);
+        past_k(o1, 1, mp, tail);
+        pin();
+    };
+    // .. and, after the copies, step 0's of the next piece (nmp) while step 1 multiplies.
+    auto back = [&](int nmp, bool next, bool tail, auto copy) {
+        copy();
+        if (next) {
+            xc = next3(xc, P6_XB);
+            wc = next4(wc, PF_WBYTES);
+            sc = (nmp & 3) == 0 ? next3(sc, PF_SBYTES) : sc;
+            read_a(o0, 0, nmp);
+            read_b(o0, 0, 0);
+            read_b(o0, 0, 1);
+            read_scales();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mul(o1, K1{}, 0, false);
+        mul(o1, K1{}, 0, true);
+        mul(o1, K1{}, 1, false);
+        mul(o1, K1{}, 1, true);
+        __builtin_amdgcn_sched_barrier(0);
+        if (next) past_k(o0, 0, nmp, tail);
+        use_scales();
+        pin();
+    };
+    // This wave's copies but the newest have landed (activations: all but the n of one piece;
+    // weights: all but two pieces', 8 copies and 4 more if one of them begins a scale group),
+    // then the barrier: piece st + 1 is in LDS and every wave holds piece st in registers.
+    auto wait_x = [&](int n) {  // n <= the wave's copies of a piece: 1, 3, 5 or 6 by the tile's 32-row groups
+        if (n >= 5) {
+            if (n == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else {
+            if (n == 3) asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+    };
+    auto wait_w = [&](bool group) {
+        if (group) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    auto x_class = [&](int rows) { return rows > 96 ? 6 : rows > 64 ? 5 : rows > 32 ? 3 : 1; };
+
+    Tile cur = tile(tl), nxt = cur;
+    int ps = 0;         // the current tile's bias and permutation slot
+    bool fresh = true;  // nothing of the current tile is in flight yet
+    for (;;) {
+        if (fresh) {  // start the stream: the first tile, or a tile after rows too short to run on
+            copy_perm(cur, ps);
+            pf_wait(0);
+            set_x(cur, ps);
+            set_w(cur);
+            for (int i = 0; i < 4 && i < MP; ++i) {
+                if (xw) {
+                    if (i < 3) issue_x(cur, i, ps);
+                } else {
+                    issue_w(i);
+                }
+                if (i < 3) next_x();
+                next_w(i, i == MP - 1);
+            }
+            pf_wait(0);
+            read_a(o0, 0, 0);
+            read_b(o0, 0, 0);
+            read_b(o0, 0, 1);
+            past_k(o0, 0, 0, true);
+            read_scales();
+            use_scales();
+            fresh = false;
+        }
+        nsub = (cur.rows - 64 * wt + 31) >> 5;
+        nsub = cur.nt * (PF_BN / 16) + 4 * wn >= N / 16 || nsub < 0 ? 0 : (nsub > 2 ? 2 : nsub);
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+
+        // Piece st multiplies while the copies run ahead, activations by 3 pieces, weights by 4,
+        // past the tile's end those of the next tile. The epilogue needs no stage, so the stream
+        // runs on under it.
+        bool more = false;  // the next tile is known and runs on in the stream
+        if (stream) {
+            int grabbed = 0;
+            const int xn = x_class(cur.rows);
+            for (int st = 0; st < MP - 4; ++st) {
+                front(st, false);
+                if (xw) wait_x(xn);
+                else wait_w(((st + 2) & 3) == 0 || ((st + 3) & 3) == 0);
+                if (st < 3) {  // the next tile: asked for, announced, read
+                    if (st == 0) {
+                        if (tid == 0) grabbed = R + __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    } else if (st == 1) {
+                        if (tid == 0) s_next = grabbed;
+                    } else {
+                        tl = uniform(s_next);
+                        more = tl < total;
+                        if (more) {
+                            nxt = tile(tl);
+                            copy_perm(nxt, ps ^ 1);
+                        }
+                    }
+                }
+                back(st + 1, true, false, [&]() {
+                    if (xw) issue_x(cur, st + 3, ps);
+                    else issue_w(st + 4);
+                    next_x();
+                    next_w(st + 4, st + 4 == MP - 1);
+                });
+            }
+#pragma unroll
+            for (int e = 4; e >= 1; --e) {  // the last four pieces, st = MP - e
+                const int st = MP - e;
+                front(st, e == 1);
+                if (e > 1 || more) {
+                    // (waits for all of a piece that may be absent or of another size: a few stricter ones a tile)
+                    if (xw) {
+                        if (e > 2) wait_x(xn);
+                        else pf_wait(0);
+                    } else if (more || e == 4) {
+                        wait_w(e == 2);  // then the next tile's pieces 0 (a group's first) and 1 are newer
+                    } else {
+                        pf_wait(0);
+                    }
+                }
+                back(e == 1 ? 0 : st + 1, e > 1 || more, e == 2, [&]() {
+                    if (xw) {
+                        if (e == 4) {
+                            issue_x(cur, MP - 1, ps);
+                        } else if (more) {
+                            if (e == 3) set_x(nxt, ps ^ 1);
+                            issue_x(nxt, 3 - e, ps ^ 1);
+                        }
+                    } else if (more) {
+                        if (e == 4) set_w(nxt);
+                        issue_w(4 - e);
+                    }
+                    next_x();
+                    next_w(4 - e, false);
+                });
+            }
+        } else {
+            for (int st = 0; st < MP; ++st) {
+                front(st, true);
+                if (st + 1 < MP) {
+                    pf_wait(0);
+                }
+                back(st + 1, st + 1 < MP, true, [&]() {
+                    if (xw && st + 3 < MP) issue_x(cur, st + 3, ps);
+                    if (!xw && st + 4 < MP) issue_w(st + 4);
+                    next_x();
+                    next_w(st + 4, st + 4 == MP - 1);
+                });
+            }
+        }
+
+        // Epilogue, in registers. acc[rb][b][4u + i] is row 32 rb + 8u + 4q + i of the wave's 64,
+        // token 64 wt + 32 b + rr: lane halves hold the halves of a token's run of rows, and a
+        // swap of column 1 of the lower lanes with column 0 of the upper ones
+        // (v_permlane32_swap) gives lane l all of token 64 wt + l's.
+        const int tk = 64 * wt + lane;
+        const uint8_t* bias = smem + P6_BOFF + 1024 * ps;
+        auto rows4 = [&](int rb, int u, int b) {  // the lane's 4 rows with their bias
+            const int c = 64 * wn + 32 * rb + 8 * u + 4 * q;
+            v4f v = v4f{acc[rb][b][4 * u], acc[rb][b][4 * u + 1], acc[rb][b][4 * u + 2], acc[rb][b][4 * u + 3]};
+            if (p.b_off >= 0) v += bias_value(*reinterpret_cast<const u32x4*>(bias + c * bes), p.L.bias_dtype);
+            return v;
+        };
+        if (nsub > 0) {
+            if constexpr (GATE_UP) {  // the wave's 64 rows are one 32-value block of h: its fp6 terms to the row's record
+                float v[32];
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const v4f a = rows4(rb, u, 0), b = rows4(rb, u, 1);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const float h0 = swiglu_oai_fast(p.L, a[2 * i], a[2 * i + 1]);
+                            const float h1 = swiglu_oai_fast(p.L, b[2 * i], b[2 * i + 1]);
+                            const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(h0), __float_as_uint(h1), false, false);
+                            v[16 * rb + 4 * u + i] = __uint_as_float(s[0]);
+                            v[16 * rb + 4 * u + 2 + i] = __uint_as_float(s[1]);
+                        }
+                    }
+                if (tk < cur.rows) {
+                    uint32_t hi[6], lo[6];
+                    const uint32_t scl = fp6_terms(v, hi, lo);
+                    uint8_t* rec = p.qout + (int64_t)(cur.row0 + tk) * p.out_stride + (int64_t)cur.nt * PF_QREC;
+                    *reinterpret_cast<uint4*>(rec + 48 * wn) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                    *reinterpret_cast<uint4*>(rec + 48 * wn + 16) = make_uint4(hi[4], hi[5], lo[0], lo[1]);
+                    *reinterpret_cast<uint4*>(rec + 48 * wn + 32) = make_uint4(lo[2], lo[3], lo[4], lo[5]);
+                    rec[PF_QSCALE + wn] = (uint8_t)scl;
+                }
+            } else {
+                const int64_t asg = *reinterpret_cast<const int*>(smem + P6_POFF + 512 * ps + 4 * tk);
+                uint16_t* dst = p.out + asg * N + PF_BN * cur.nt + 64 * wn;
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const v4f a = rows4(rb, u, 0), b = rows4(rb, u, 1);
+                        const auto s0 = __builtin_amdgcn_permlane32_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
+                        const auto s1 = __builtin_amdgcn_permlane32_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
+                        if (tk < cur.rows && PF_BN * cur.nt + 64 * wn + 32 * rb + 8 * u < N)
+                            *reinterpret_cast<uint4*>(dst + 32 * rb + 8 * u) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+                    }
+            }
+        } else if constexpr (GATE_UP) {  // blocks past the row's end: zero codes with a unit scale
+            const int cb = 4 * cur.nt + wn;
+            if (32 * cb >= N / 2 && tk < cur.rows) {
+                uint8_t* rec = p.qout + (int64_t)(cur.row0 + tk) * p.out_stride + (int64_t)cur.nt * PF_QREC;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4*>(rec + 48 * wn + 16 * i) = make_uint4(0u, 0u, 0u, 0u);
+                rec[PF_QSCALE + wn] = 127;
+            }
+        }
+        if (more) {
+            cur = nxt;
+            ps ^= 1;
+            continue;
+        }
+        if (stream) return;  // no tile left
+        if (tid == 0) s_next = R + __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        tl = uniform(s_next);
+        if (tl >= total) return;
+        cur = tile(tl);
+        xg = wg = sg = xc = wc = sc = 0;
+        fresh = true;
+        __syncthreads();  // s_next is read and every wave is done with the tile before it is refilled
     }
 }
 
@@ -798,12 +1183,13 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
                        nent, table, ctr);
     TSA_LAUNCH_CHECK();
 
-    for (const void* f : {reinterpret_cast<const void*>(pf_gemm_kernel<true, false>),
-                          reinterpret_cast<const void*>(pf_gemm_kernel<false, false>),
-                          reinterpret_cast<const void*>(pf_gemm_kernel<true, true>),
-                          reinterpret_cast<const void*>(pf_gemm_kernel<false, true>)}) {
-        const hipError_t e = ensure_dynamic_lds(f, PF_LDS);
-        TSA_REQUIRE(e == hipSuccess, TSA_ERR_HIP, "hipFuncSetAttribute(LDS %d): %s", PF_LDS, hipGetErrorString(e));
+    const bool q6 = L.prefill_mfma == TSA_PREFILL_FP6;
+    const void* f_gu = q6 ? reinterpret_cast<const void*>(pf6_gemm_kernel<true>) : reinterpret_cast<const void*>(pf_gemm_kernel<true>);
+    const void* f_dn = q6 ? reinterpret_cast<const void*>(pf6_gemm_kernel<false>) : reinterpret_cast<const void*>(pf_gemm_kernel<false>);
+    const int lds = q6 ? P6_LDS : PF_LDS;
+    for (const void* f : {f_gu, f_dn}) {
+        const hipError_t e = ensure_dynamic_lds(f, lds);
+        TSA_REQUIRE(e == hipSuccess, TSA_ERR_HIP, "hipFuncSetAttribute(LDS %d): %s", lds, hipGetErrorString(e));
     }
     const int grid = (num_cus() / 8) * 8;
     PfGemm g{};
@@ -814,7 +1200,7 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
     g.perm = perm;
     g.ctr = ctr;
     g.k = k;
-    const bool q6 = L.prefill_mfma == TSA_PREFILL_FP6;
+    void* args[] = {&g};
     uint8_t* xq = ws + w.xq;
     if (q6) {  // x as fp6 records
         const int64_t threads = T * 4 * ((H + 127) / 128);
@@ -838,9 +1224,7 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
     g.b_off = L.gate_bias_off;
     g.tile_bytes = 16 * (int64_t)H / 2;
     g.stile_bytes = mx_tile_scale_bytes(H);
-    if (q6) hipLaunchKernelGGL((pf_gemm_kernel<true, true>), dim3(grid), dim3(PF_THREADS), PF_LDS, stream, g);
-    else hipLaunchKernelGGL((pf_gemm_kernel<true, false>), dim3(grid), dim3(PF_THREADS), PF_LDS, stream, g);
-    TSA_LAUNCH_CHECK();
+    TSA_HIP_CHECK(hipLaunchKernel(f_gu, dim3(grid), dim3(PF_THREADS), args, lds, stream));
     // down: [H, I] -> yk
     g.src = ws + w.h;
     g.src_rows = T * k;
@@ -856,9 +1240,7 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
     g.b_off = L.down_bias_off;
     g.tile_bytes = 16 * (int64_t)I / 2;
     g.stile_bytes = mx_tile_scale_bytes(I);
-    if (q6) hipLaunchKernelGGL((pf_gemm_kernel<false, true>), dim3(grid), dim3(PF_THREADS), PF_LDS, stream, g);
-    else hipLaunchKernelGGL((pf_gemm_kernel<false, false>), dim3(grid), dim3(PF_THREADS), PF_LDS, stream, g);
-    TSA_LAUNCH_CHECK();
+    TSA_HIP_CHECK(hipLaunchKernel(f_dn, dim3(grid), dim3(PF_THREADS), args, lds, stream));
 
     return pf_combine(yk, idx, weights, expert_slot, E, n_slots, T, k, H, y, y_dtype, stream);
 }
