@@ -10,7 +10,7 @@ import torch
 from oracle import gguf as og
 from oracle import mxfp4 as omx
 from tests.helpers import bits_equal, dev_u8
-from tinyserve_amd import ops, synth
+from tinyserve_amd import _lib, ops, synth
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden", "dequant_golden.npz")
@@ -90,3 +90,30 @@ def test_mxfp4_dequant_random_vs_oracle(N, G):
     assert bits_equal(out.cpu().numpy(), ref)
     out_bf = ops.mxfp4_dequant(torch.from_numpy(blocks).cuda(), torch.from_numpy(scales).cuda(), torch.bfloat16)
     assert np.array_equal(out_bf.float().cpu().numpy(), omx.bf16_round(ref))
+
+
+@pytest.mark.parametrize("gtype", [8, 12, 13, 14])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gguf_dequant_output_4byte_aligned(gtype, dtype):
+    """Outputs on a 4-byte boundary (not 16) take the element stores, with the same values."""
+    n = 256 * 5
+    data = synth.make_gguf(np.random.default_rng(gtype), gtype, n)
+    d = dev_u8(data)
+    want = ops.gguf_dequant(d, gtype, (n,), dtype=dtype)
+    buf = torch.zeros(n + 16, dtype=dtype, device="cuda")
+    lib, out = _lib.load(), buf[2 : 2 + n]
+    _lib.check(lib.tsa_gguf_dequant(gtype, d.data_ptr(), d.numel(), n, out.data_ptr(), _lib.tsa_dtype(dtype),
+                                    _lib.stream_handle(d.device)))
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16)) and not buf[:2].any() and not buf[2 + n :].any()
+
+
+@pytest.mark.parametrize("dtype,offset", [(torch.bfloat16, 1), (torch.float16, 5), (torch.float32, 3)])
+def test_mxfp4_dequant_unaligned_output(dtype, offset):
+    rng = np.random.default_rng(offset)
+    blocks = torch.from_numpy(rng.integers(0, 256, size=(33, 5, 16), dtype=np.uint8)).cuda()
+    scales = torch.from_numpy(rng.integers(110, 140, size=(33, 5), dtype=np.uint8)).cuda()
+    want = ops.mxfp4_dequant(blocks, scales, dtype=dtype)
+    buf = torch.zeros(want.numel() + 16, dtype=dtype, device="cuda")
+    out = buf[offset : offset + want.numel()]
+    ops.mxfp4_dequant(blocks, scales, dtype=dtype, out=out)
+    assert torch.equal(out.view_as(want), want) and not buf[:offset].any() and not buf[offset + want.numel() :].any()

@@ -59,6 +59,14 @@ __device__ __forceinline__ void k_scale_min(const uint32_t s[3], int j, uint32_t
     }
 }
 
+// The same for a sub-block that is only known at run time (no indexed field bytes): h is the
+// super-block's first 16 bytes.
+__device__ __forceinline__ void k_scale_min_at(const uint32_t* h, uint32_t u, uint32_t& sc, uint32_t& m) {
+    const uint32_t sh = 8 * (u & 3), s0 = h[1] >> sh, s1 = h[2] >> sh, s2 = h[3] >> sh;
+    sc = u < 4 ? s0 & 63u : (s2 & 15u) | ((s0 >> 2) & 0x30u);
+    m = u < 4 ? s1 & 63u : ((s2 >> 4) & 15u) | ((s1 >> 2) & 0x30u);
+}
+
 template <int TYPE, int A>
 __device__ __forceinline__ void decode_unit(const uint8_t* b, int u, float v[32]);
 

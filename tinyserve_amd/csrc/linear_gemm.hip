@@ -165,17 +165,6 @@ __device__ __forceinline__ void lg_split(const float (&v)[16], uint32_t (&hi)[8]
     }
 }
 
-// Scale and min of sub-block u (a lane's own) of a K-quant header (k_scale_min with a
-// variable index).
-__device__ __forceinline__ void lg_scale_min(const uint32_t* h, uint32_t u, float& a, float& c) {
-    const uint32_t sh = 8 * (u & 3), s0 = h[1] >> sh, s1 = h[2] >> sh, s2 = h[3] >> sh;
-    const bool lowh = u < 4;
-    const uint32_t sc = lowh ? s0 & 63u : (s2 & 15u) | ((s0 >> 2) & 0x30u);
-    const uint32_t m = lowh ? s1 & 63u : ((s2 >> 4) & 15u) | ((s1 >> 2) & 0x30u);
-    a = f16_bits_to_f32(h[0] & 0xFFFFu) * (float)sc;
-    c = f16_bits_to_f32(h[0] >> 16) * (float)m;
-}
-
 // Unit i (0 .. 3) of the step as A operands: hi[4 s ..], lo[4 s ..] for K step s (lo only for
 // GGUF weights). H: the half super-block of an aligned K-quant row.
 template <int F, bool SD, int H>
@@ -210,16 +199,14 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
             const uint32_t* hd = SD ? R + (F == 12 ? 8 : 12) * i : R;
             const uint32_t* qs = SD ? hd + 4 : R + 4 + 4 * (i >> 1);
             const uint32_t* qh = SD ? hd + 8 : R + 12;
-            float a, c;
+            uint32_t sc, m;
             if constexpr (SD) {
-                lg_scale_min(hd, u, a, c);
+                k_scale_min_at(hd, u, sc, m);
             } else {
                 const uint32_t s3[3] = {hd[1], hd[2], hd[3]};
-                uint32_t sc, m;
                 k_scale_min(s3, 4 * H + i, sc, m);
-                a = f16_bits_to_f32(hd[0] & 0xFFFFu) * (float)sc;
-                c = f16_bits_to_f32(hd[0] >> 16) * (float)m;
             }
+            const float a = f16_bits_to_f32(hd[0] & 0xFFFFu) * (float)sc, c = f16_bits_to_f32(hd[0] >> 16) * (float)m;
             const uint32_t sh = 4 * (u & 1);
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
