@@ -27,15 +27,13 @@
 // the codes that half reads) come in one step ahead into one of two tiles and areas, 77 KB
 // of LDS at most, so two workgroups share a CU.
 //
-// gf_gemm_kernel (Q8_0, and K-quant rows that straddle super-blocks): K in pieces of 256
-// values (one super-block of each row, or 8 Q8_0 blocks), up to 154 KB of LDS, one workgroup
-// per CU: the activations into one of two tiles as the previous piece starts, the raw blocks
-// into a ring of areas ahead of their piece. Where K is not a multiple of 256 (hidden 2880),
-// a K-quant row starts inside a super-block (GGUF stores a matrix as one run of blocks) and a
-// piece of it covers the end of one super-block and the start of the next: that variant keeps
-// each row's super-blocks in a ring of areas, one new super-block per piece, and decodes
-// every 32-value unit from whichever super-block holds it; the last piece of a row is
-// partial, its units past K zeroed.
+// gf_gemm_kernel (Q8_0): K in pieces of 256 values (8 blocks of each row), one workgroup per
+// CU: the activations into one of two tiles and the raw blocks into one of two areas as the
+// previous piece starts.
+//
+// gf_reg_kernel (K-quant rows where K is not a multiple of 256, hidden 2880: GGUF stores a
+// matrix as one run of blocks, so a row starts inside a super-block): whole super-blocks from
+// memory straight into registers, two workgroups per CU.
 //
 // Semantics: tinyserve/expert_pipeline.py:166-239 (group by expert, batched forward,
 // weighted scatter), tinyserve/ggml_forward.py:117-151 (bf16 weights, F.linear,
@@ -71,30 +69,16 @@ struct GfEntry {
     int slot, row0, rows, pad;
 };
 
-// Raw bytes of one row's K piece (a raw group): a K-quant super-block, or 8 Q8_0 blocks.
+// Raw bytes of one row's 256 values (a raw group): a K-quant super-block, or 8 Q8_0 blocks.
 template <int TY> struct GfType { static constexpr int PB = TY == 8 ? 272 : TY == 12 ? 144 : TY == 13 ? 176 : 210; };
-// Alignment of a raw group in LDS, which keeps its global address modulo 16: the K-quant
-// 4/5-bit super-blocks (144 / 176 bytes) stay 16-aligned, Q6_K / Q8_0 2-aligned (the host
-// requires pool, slot size and offsets to keep that).
-template <int TY> constexpr int gf_align() { return TY == 12 || TY == 13 ? 16 : 2; }
-// 16-byte chunks of a group's window: from the boundary at or below the group (up to 14
-// bytes before it when 2-aligned) to its end, rounded up to an odd count: the 32 rows a
-// wave's lanes decode from then sit 4 (mod 8) dwords apart and spread over 16 bank groups
-// (an even count halves that or worse: Q6_K's 14 chunks cost its kernel 8% against 15).
-template <int TY> constexpr int gf_nch() { return ((GfType<TY>::PB + (gf_align<TY>() == 16 ? 0 : 14) + 15) / 16) | 1; }
-// gf_gemm_kernel's raw areas, each the 128 rows' windows of one group. Plain (Q8_0): the
-// piece in use and the next (three areas of its windows would not fit beside the activation
-// tiles). Straddling (SD): a piece reads two groups of its row, and one or two more areas
-// take the groups ahead (Q6_K: one; its windows leave room for three areas only).
-template <int TY, bool SD> constexpr int gf_areas() { return SD ? (TY == 14 ? 3 : 4) : 2; }
-template <int TY> constexpr int gf_raw() { return GF_BN * gf_nch<TY>() * 16; }
-template <int TY, bool SD> constexpr int gf_lds() {
-    return GF_ROFF + gf_areas<TY, SD>() * gf_raw<TY>() > GF_STAGE ? GF_ROFF + gf_areas<TY, SD>() * gf_raw<TY>()
-                                                                  : GF_STAGE;
-}
-static_assert(gf_lds<8, false>() <= 160 * 1024 && gf_lds<12, true>() <= 160 * 1024 &&
-                  gf_lds<13, true>() <= 160 * 1024 && gf_lds<14, true>() <= 160 * 1024,
-              "LDS per workgroup");
+// gf_gemm_kernel: 16-byte chunks of a group's window, from the boundary at or below the group
+// (2-byte aligned: the window keeps its global address modulo 16, the host requires pool, slot
+// size and offsets to keep the 2) to its end, rounded up to an odd count: the 32 rows a wave's
+// lanes decode from then sit 4 (mod 8) dwords apart and spread over 16 bank groups.
+constexpr int GF_NCH = ((GfType<8>::PB + 14 + 15) / 16) | 1;
+constexpr int GF_RAW = GF_BN * GF_NCH * 16;  // the 128 rows' windows of one group; two areas
+constexpr int GF_LDS = GF_ROFF + 2 * GF_RAW > GF_STAGE ? GF_ROFF + 2 * GF_RAW : GF_STAGE;
+static_assert(GF_LDS <= 160 * 1024, "LDS per workgroup");
 
 struct GfGemm {
     const uint8_t* pool;
@@ -137,15 +121,15 @@ __device__ __forceinline__ uint32_t gf_group_byte(int row, int q, int KU) {
     else return (((uint32_t)row * (uint32_t)KU >> 3) + (uint32_t)q) * (uint32_t)GfType<TY>::PB;
 }
 
-// Raw group q's windows of the tile's 128 weight rows into LDS: pair i = (row i / NCH,
+// Q8_0 group q's windows of the tile's 128 weight rows into LDS: pair i = (row i / NCH,
 // chunk i % NCH) lands at raw + 16 i, so one wave instruction fills 1 KB. The buffers start
 // at the 16-byte boundary at or below each matrix (m0 / m1 bytes before it) and end at the
 // boundary at or above its end, and a window starts at the boundary at or below its group,
 // so every copy reads 16 whole aligned bytes; rows past the matrix read zero (buffer range).
-template <int TY, bool GU>
+template <bool GU>
 __device__ __forceinline__ void gf_issue_raw(const v4i_t& r0, const v4i_t& r1, uint32_t m0, uint32_t m1, int n0,
                                              int p, int KU, uint32_t raw, int wave, int lane) {
-    constexpr int NCH = gf_nch<TY>(), TOT = GF_BN * NCH;
+    constexpr int NCH = GF_NCH, TOT = GF_BN * NCH;
     for (int ii = wave; 64 * ii < TOT; ii += GF_THREADS / 64) {
         const int q = 64 * ii + lane;
         if (q < TOT) {
@@ -153,7 +137,7 @@ __device__ __forceinline__ void gf_issue_raw(const v4i_t& r0, const v4i_t& r1, u
             const bool up = GU && r >= 64;
             const int row = GU ? n0 + (r & 63) : n0 + r;
             const uint32_t m = up ? m1 : m0;
-            const uint32_t voff = ((m + gf_group_byte<TY>(row, p, KU)) & ~15u) + 16u * (uint32_t)c;
+            const uint32_t voff = ((m + gf_group_byte<8>(row, p, KU)) & ~15u) + 16u * (uint32_t)c;
             if (up) gf_dma(r1, voff, raw + 1024u * (uint32_t)ii);
             else gf_dma(r0, voff, raw + 1024u * (uint32_t)ii);
         }
@@ -169,16 +153,16 @@ __device__ __forceinline__ void gf_issue_raw(const v4i_t& r0, const v4i_t& r1, u
 // rounding, fused or not); Q6_K (d*sc) * (q - 32), here as (d*sc/4) times the signed byte
 // 4 (q - 32) (q ^ 32 is q - 32 as a 6-bit two's-complement field, and two more bits to the
 // left make the byte's sign), exact like the reference's product, signed zeros included.
-// HALF: sb is a half window (gf_step_kernel) holding only what units 4h .. 4h + 3 (h = u / 4)
+// A K-quant's sb is a half window (gf_step_kernel) holding only what units 4h .. 4h + 3 (h = u / 4)
 // read, at the offsets gf_half_chunk lays out: Q4_K / Q5_K keep the header (and Q5_K's high
 // bits) and take the half's 64 bytes of codes right after; Q6_K's half window is the half's
 // low codes (block bytes 64 h ..), high codes (128 + 32 h ..) at +80 and scales and d
 // (192 ..) at -64, each from sb.
-template <int TY, bool HALF = false>
+template <int TY>
 __device__ __forceinline__ void gf_decode_a(const uint8_t* sb, int u, int g, uint32_t (&o)[8]) {
     if constexpr (TY == 12 || TY == 13) {  // sb is 16-byte aligned
         const u32x4 hdr = *reinterpret_cast<const u32x4*>(sb);
-        const uint8_t* qs = sb + (TY == 12 ? 16 : 48) + 32 * (HALF ? (u >> 1) & 1 : u >> 1);
+        const uint8_t* qs = sb + (TY == 12 ? 16 : 48) + 32 * ((u >> 1) & 1);
         const uint2 q0 = *reinterpret_cast<const uint2*>(qs + 8 * g), q1 = *reinterpret_cast<const uint2*>(qs + 16 + 8 * g);
         const uint32_t q[4] = {q0.x, q0.y, q1.x, q1.y};
         uint32_t hb[4] = {0u, 0u, 0u, 0u};
@@ -196,6 +180,7 @@ __device__ __forceinline__ void gf_decode_a(const uint8_t* sb, int u, int g, uin
         for (int w = 0; w < 4; ++w) {
             uint32_t qq = (q[w] >> sh) & 0x0F0F0F0Fu;
             if constexpr (TY == 13) qq |= ((hb[w] >> u) & 0x01010101u) << 4;
+            asm("" : "+v"(qq));  // masked once for its four bytes
             o[2 * w] = pack_bf16x2(a * (float)(qq & 0xFFu) - c, a * (float)((qq >> 8) & 0xFFu) - c);
             o[2 * w + 1] = pack_bf16x2(a * (float)((qq >> 16) & 0xFFu) - c, a * (float)(qq >> 24) - c);
         }
@@ -206,15 +191,10 @@ __device__ __forceinline__ void gf_decode_a(const uint8_t* sb, int u, int g, uin
         const uint32_t* wb = reinterpret_cast<const uint32_t*>(sb - ob);
         auto ld4 = [&](int off, uint32_t (&w)[4]) {  // dwords 2g, 2g + 1, 2g + 4, 2g + 5 of the 32 bytes at sb + off
             const int b0 = (off >> 2) + 2 * g;
-            uint32_t t0, t1, t2, t4, t5, t6;  // at most the ninth: inside the block or half window
-            if constexpr (HALF) {  // a half window starts at the dword of its block (wb), 16-byte aligned: 8-byte reads
-                const uint2* w2 = reinterpret_cast<const uint2*>(wb + b0);
-                const uint2 p0 = w2[0], p1 = w2[1], p2 = w2[2], p3 = w2[3];
-                t0 = p0.x, t1 = p0.y, t2 = p1.x, t4 = p2.x, t5 = p2.y, t6 = p3.x;
-            } else {
-                t0 = wb[b0], t1 = wb[b0 + 1], t2 = wb[b0 + 2];
-                t4 = wb[b0 + 4], t5 = wb[b0 + 5], t6 = wb[b0 + 6];
-            }
+            // a half window starts at the dword of its block (wb), 16-byte aligned: 8-byte reads
+            const uint2* w2 = reinterpret_cast<const uint2*>(wb + b0);
+            const uint2 p0 = w2[0], p1 = w2[1], p2 = w2[2], p3 = w2[3];
+            const uint32_t t0 = p0.x, t1 = p0.y, t2 = p1.x, t4 = p2.x, t5 = p2.y, t6 = p3.x;
             w[0] = __builtin_amdgcn_alignbyte(t1, t0, ob);
             w[1] = __builtin_amdgcn_alignbyte(t2, t1, ob);
             w[2] = __builtin_amdgcn_alignbyte(t5, t4, ob);
@@ -224,18 +204,19 @@ __device__ __forceinline__ void gf_decode_a(const uint8_t* sb, int u, int g, uin
             const uint32_t a = ob + (uint32_t)off;
             return (wb[a >> 2] >> (8u * (a & 3u))) & 0xFFFFu;
         };
-        const int hh = u >> 2, t = u & 3;
+        const int t = u & 3;
         uint32_t ql[4], qh[4];
-        ld4(HALF ? 32 * (t & 1) : 64 * hh + 32 * (t & 1), ql);
-        ld4(HALF ? 80 : 128 + 32 * hh, qh);
-        const uint32_t scw = ld16((HALF ? 128 : 192) + 2 * u);
-        const float d = f16_bits_to_f32(ld16(HALF ? 144 : 208));
+        ld4(32 * (t & 1), ql);
+        ld4(80, qh);
+        const uint32_t scw = ld16(128 + 2 * u);
+        const float d = f16_bits_to_f32(ld16(144));
         const float d0 = 0.25f * (d * (float)(int8_t)(scw & 0xFF)), d1 = 0.25f * (d * (float)(int8_t)(scw >> 8));
         const int shl = 4 * (t >> 1), shh = 2 * t;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const uint32_t qq = ((ql[w] >> shl) & 0x0F0F0F0Fu) | (((qh[w] >> shh) & 0x03030303u) << 4);
-            const uint32_t y = (qq ^ 0x20202020u) << 2;  // four signed bytes 4 (q - 32)
+            uint32_t y = (qq ^ 0x20202020u) << 2;  // four signed bytes 4 (q - 32)
+            asm("" : "+v"(y));
             const float dd = w < 2 ? d0 : d1;            // values below 16 take sc[2u], the rest sc[2u + 1]
             o[2 * w] = pack_bf16x2(dd * (float)(int8_t)(y & 0xFFu), dd * (float)(int8_t)((y >> 8) & 0xFFu));
             o[2 * w + 1] = pack_bf16x2(dd * (float)(int8_t)((y >> 16) & 0xFFu), dd * (float)(int8_t)(y >> 24));
@@ -318,7 +299,7 @@ __device__ __forceinline__ void gf_store_tile(const GfGemm& p, const GfEntry& en
     }
 }
 
-template <int TY, bool GU, bool SD>
+template <bool GU>
 __global__ void __launch_bounds__(GF_THREADS, 1) gf_gemm_kernel(GfGemm p) {
     extern __shared__ __align__(16) uint8_t smem[];
     // Work id w = (entry, column tile) of this workgroup. Workgroups are dealt round the 8
@@ -345,21 +326,12 @@ __global__ void __launch_bounds__(GF_THREADS, 1) gf_gemm_kernel(GfGemm p) {
                 rs1 = gf_desc(mat1 - mis1, (p.w_bytes + mis1 + 15) & ~15ll);
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
     const uint32_t raw = lds0 + GF_ROFF;
-    constexpr int RA = gf_areas<TY, SD>(), RAW = gf_raw<TY>();
-    // raw groups per row (a straddling piece also reads the next group) and how many of the
-    // newest may still fly when a piece starts
-    const int NG = SD ? P + 1 : P;
-    constexpr int OUT = RA - 2 - (SD ? 1 : 0);
-    static_assert(OUT == 0 || OUT == 1, "raw groups in flight at a piece's start");
-
     // Activation tiles: row r holds sorted row r's piece as 32 chunks of 16 bytes, chunk c in
     // slot c ^ (r % 32), so the 32 rows of an MFMA operand read fall on distinct banks. They
     // arrive by buffer-to-LDS copies: wave w's copy i fills rows 8w + 2i and 8w + 2i + 1 (1 KB,
     // lane l: row 8w + 2i + l / 32, slot l % 32, so it reads chunk (l % 32) ^ row % 32).
     // Rows past the tile's read zeros (an offset past the buffer's end).
-    // Columns past K (the last piece of a row when K % 256 != 0) read zeros as well. Only the
-    // straddling variants and Q8_0 can have such a piece (a plain K-quant kernel has K % 256 == 0).
-    constexpr bool TAILS = SD || TY == 8;
+    // Columns past K (the last piece of a row when K % 256 != 0) read zeros as well.
     const v4i_t rx = gf_desc(reinterpret_cast<const uint8_t*>(p.src), p.src_bytes);
     uint32_t xo[4];
     int xc[4];  // the first column of this lane's chunk in piece 0
@@ -376,23 +348,21 @@ __global__ void __launch_bounds__(GF_THREADS, 1) gf_gemm_kernel(GfGemm p) {
     }
     auto issue_x = [&](int pc) {
         const uint32_t t = lds0 + (uint32_t)(pc & 1) * GF_XB + (uint32_t)(8 * wave) * GF_RS;
-        const bool tail = TAILS && (K & (GF_KP - 1)) && pc == P - 1;  // wave-uniform
+        const bool tail = (K & (GF_KP - 1)) && pc == P - 1;  // wave-uniform
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t o = tail && GF_KP * pc + xc[i] >= K ? 0x80000000u : xo[i] + (uint32_t)pc * (2 * GF_KP);
             gf_dma(rx, o, t + (uint32_t)(2 * i) * GF_RS);
         }
     };
-    // this wave's raw copies per piece: instructions ii = wave, wave + 8, .. below NI
-    constexpr int NI = (GF_BN * gf_nch<TY>() + 63) / 64, RWA = (NI + 7) / 8, RWB = NI / 8;
-    const bool rw_more = wave < NI % 8;
+    auto issue_raw = [&](int pc) {
+        gf_issue_raw<GU>(rs0, rs1, mis0, mis1, n0, pc, KU, raw + (uint32_t)(pc & 1) * GF_RAW, wave, lane);
+    };
 
     // This lane's weight row: tile row 32 wr + rr (gate_up: rows 64.. are the up rows).
     const int trow = 32 * wr + rr;
     const int drow = GU ? n0 + (trow & 63) : n0 + trow;
-    constexpr int NCH = gf_nch<TY>();
     const uint32_t dmis = GU && trow >= 64 ? mis1 : mis0;
-    const int ph = SD ? (int)(((uint32_t)drow * (uint32_t)KU) & 7u) : 0;  // the row's first unit in its super-block
 
     v16f_t acc[2];
 #pragma unroll
@@ -400,46 +370,30 @@ __global__ void __launch_bounds__(GF_THREADS, 1) gf_gemm_kernel(GfGemm p) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
 
-    // Piece pc's activations sit in tile pc % 2 and raw group q in area q % RA. As piece pc
-    // starts, the copies of piece pc + 1's activations and then of group pc + RA - 1 go out
-    // (into the area group pc - 1 left), so a group flies for RA - 2 pieces (plain) or
-    // RA - 3 (straddling: piece pc reads groups pc and pc + 1). A tile or area is rewritten
-    // one piece after it was last read, with the barrier of the piece between. Every load
-    // here is an inline-assembly copy (the compiler counts none of them), so the waits are
-    // explicit: at the top of piece pc everything must have landed but the newest OUT groups
-    // (the RWA or RWB instructions per group of this wave).
+    // Piece pc's activations and raw group sit in tile and area pc % 2, rewritten one piece after
+    // they were last read, with the barrier of the piece between. Every load here is an
+    // inline-assembly copy (the compiler counts none of them), so the waits are explicit.
     issue_x(0);
-    for (int q = 0; q < RA - 1 && q < NG; ++q)
-        gf_issue_raw<TY, GU>(rs0, rs1, mis0, mis1, n0, q, KU, raw + (uint32_t)q * RAW, wave, lane);
+    issue_raw(0);
     for (int pc = 0; pc < P; ++pc) {
         const uint8_t* xt = smem + (pc & 1) * GF_XB;
-        if (OUT == 1 && pc + RA - 2 < NG) {
-            if (rw_more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RWA) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RWB) : "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // piece pc is in LDS; tile and area (pc + 1) % 2 are free
+        if (pc + 1 < P) {
+            issue_x(pc + 1);
+            issue_raw(pc + 1);
         }
-        __syncthreads();  // piece pc's raw groups and activations are in LDS; tile (pc + 1) % 2 and area (pc - 1) % RA are free
-        if (pc + 1 < P) issue_x(pc + 1);
-        if (pc + RA - 1 < NG)
-            gf_issue_raw<TY, GU>(rs0, rs1, mis0, mis1, n0, pc + RA - 1, KU, raw + (uint32_t)((pc + RA - 1) % RA) * RAW,
-                                 wave, lane);
         // unit uu of the half, then its two K steps (the next unit's decode can issue while
         // these MFMAs run); step j: K 16 j .. + 15 of the half, lane half g holds K 16 j + 8 g .. + 7
         const uint8_t* xr0 = xt + rr * GF_RS;  // sorted row rr (t = 0) and 32 + rr (t = 1): same swizzle
-        // this lane's window of group pc (and, straddling, of group pc + 1)
-        const uint8_t* sb0 = smem + GF_ROFF + (pc % RA) * RAW + 16 * NCH * trow +
-                             ((dmis + gf_group_byte<TY>(drow, pc, KU)) & 15u);
-        const uint8_t* sb1 = SD ? smem + GF_ROFF + ((pc + 1) % RA) * RAW + 16 * NCH * trow +
-                                      ((dmis + gf_group_byte<TY>(drow, pc + 1, KU)) & 15u)
-                                : sb0;
-        const bool tail = TAILS && (KU & 7) && pc == P - 1;  // wave-uniform: the row's last, partial piece
+        // this lane's window of group pc
+        const uint8_t* sb = smem + GF_ROFF + (pc & 1) * GF_RAW + 16 * GF_NCH * trow + ((dmis + gf_group_byte<8>(drow, pc, KU)) & 15u);
+        const bool tail = (KU & 7) && pc == P - 1;  // wave-uniform: the row's last, partial piece
 #pragma unroll
         for (int uu = 0; uu < 4; ++uu) {
             const int j = 4 * kh + uu;  // unit of the piece
-            const int v = ph + j;       // straddling: unit v % 8 of group pc + v / 8
             uint32_t av[8];
-            gf_decode_a<TY>(SD && v >= 8 ? sb1 : sb0, SD ? v & 7 : j, g, av);
+            gf_decode_a<8>(sb, j, g, av);
             if (tail && 8 * pc + j >= KU) {  // past the row's end: another row's values or zeros
 #pragma unroll
                 for (int i = 0; i < 8; ++i) av[i] = 0u;
@@ -468,7 +422,7 @@ constexpr int GF_SRS = 2 * GF_KS;        // a step's activation row: 256 bytes, 
 constexpr int GF_SXB = GF_BM * GF_SRS;   // one step activation tile; two of them
 constexpr int GF_SROFF = 2 * GF_SXB;     // then two raw areas
 
-// 16-byte chunks of a row's half window (odd, as gf_nch): Q4_K header + 4 of codes; Q5_K
+// 16-byte chunks of a row's half window (odd, as GF_NCH): Q4_K header + 4 of codes; Q5_K
 // header, high bits + 4 of codes; Q6_K 5 of low codes, 3 of high codes, 2 of scales and d
 // (+1 unused). A Q6_K window's chunks are counted from the dword at or below its block (0
 // or 2 bytes before it: the copies read 16 bytes at dword-aligned offsets), so the block
@@ -593,7 +547,7 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
 #pragma unroll
         for (int uu = 0; uu < 2; ++uu) {
             uint32_t av[8];
-            gf_decode_a<TY, true>(sb, 4 * h + 2 * khc + uu, g, av);
+            gf_decode_a<TY>(sb, 4 * h + 2 * khc + uu, g, av);
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
                 const bf16x8 A = __builtin_bit_cast(bf16x8, u32x4{av[4 * s2], av[4 * s2 + 1], av[4 * s2 + 2], av[4 * s2 + 3]});
@@ -624,18 +578,277 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
     gf_store_tile<GU>(p, en, n0, acc, smem);
 }
 
-template <int TY, bool GU, bool SD>
-const void* gf_fn() { return reinterpret_cast<const void*>(&gf_gemm_kernel<TY, GU, SD>); }
+// ---- gf_reg_kernel: K-quant matrices whose rows straddle super-blocks (K % 256 != 0)
 
-// gf_gemm_kernel runs Q8_0 (plain) and the K-quants' straddling rows
-const void* gf_pick(int t, bool gu) {
-    switch (t) {
-        case 8: return gu ? gf_fn<8, true, false>() : gf_fn<8, false, false>();
-        case 12: return gu ? gf_fn<12, true, true>() : gf_fn<12, false, true>();
-        case 13: return gu ? gf_fn<13, true, true>() : gf_fn<13, false, true>();
-        case 14: return gu ? gf_fn<14, true, true>() : gf_fn<14, false, true>();
+// Workgroup: 8 waves, a tile of 64 sorted rows x 256 weight rows (gate_up: 128 gate rows and the
+// same up rows, 16 + 16 per wave, so gate and up of an output meet in one lane's registers). A
+// wave owns its 32 rows over all of K. They are every eighth row of the tile, so they start at
+// one place ph of their super-blocks (8 KU values is a whole number of those): every wave walks
+// its rows super-block by super-block with constant shifts and scales, and the unit j of the
+// row that unit u of super-block q is, 8 q + u - ph, comes from a ring of 4 activation tiles
+// (128 values each) that covers every ph. A lane reads its half of a super-block in 5 to 8
+// 16-byte loads, all at once and a super-block ahead: a row's cache lines are fetched once (16
+// bytes per step and wave took 2.4 times as long, the lines having left L1 in between). No
+// weight goes through LDS and its 64 KB leave room for two workgroups per CU.
+// Bound by those row-divergent loads and the decode about equally (with one of them taken out
+// either gains 10 .. 15%, the matrix cores are a fifth busy). hidden = inter = 2880, 32 experts,
+// top 4, Q4_K gate / up and Q6_K down, gate_up + down in us, against pieces of 256 values staged
+// through LDS by one workgroup per CU: 40 tokens 109 + 73 -> 72 + 71, 301 tokens 236 + 142 ->
+// 149 + 135, 1023 tokens 443 + 273 -> 263 + 200.
+constexpr int GR_KS = 128;                    // values per step: half a super-block
+constexpr int GR_RS = 2 * GR_KS;              // an activation tile row: a step of a sorted row, 16 chunks
+constexpr int GR_LDS = 64 * 1024;             // the ring of activation tiles, then the staged results
+constexpr int GR_XB = GF_BM * GR_RS;          // an activation tile
+constexpr int GR_RING = 4;
+static_assert(GR_RING * GR_XB == GR_LDS, "the ring fills the LDS");
+
+// 16 bytes at p + off, dword-aligned, in one load.
+typedef __attribute__((address_space(1))) const uint8_t* gr_ptr;
+__device__ __forceinline__ void gr_ld16(gr_ptr p, int off, uint32_t* d) {
+    struct __attribute__((packed, aligned(4))) U { u32x4 v; };
+    const u32x4 v = reinterpret_cast<__attribute__((address_space(1))) const U*>(p + off)->v;
+    d[0] = v[0], d[1] = v[1], d[2] = v[2], d[3] = v[3];
+}
+
+// A super-block as lane half g holds it: of each unit the codes of values 16 g .. 16 g + 15,
+// and the scales. Dwords, and the loads of gr_load.
+template <int TY> constexpr int gr_nraw() { return TY == 12 ? 20 : TY == 13 ? 24 : 29; }
+template <int TY> constexpr int gr_nload() { return TY == 12 ? 5 : 6; }
+// A Q6_K block sits 2 bytes off a dword boundary for half the rows: its loads start at the
+// dword at or below it (a misaligned 16-byte load costs about two), gr_align puts them in place.
+template <int TY>
+__device__ __forceinline__ void gr_load(gr_ptr blk, int g, uint32_t (&R)[gr_nraw<TY>()]) {
+    if constexpr (TY == 14) blk = (gr_ptr)((uint64_t)blk & ~3ull);
+    const gr_ptr bg = blk + 16 * g;
+    if constexpr (TY == 14) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gr_ld16(bg, 32 * i, R + 4 * i);
+        gr_ld16(bg, 128, R + 16);
+        gr_ld16(bg, 160, R + 20);
+    } else {
+        constexpr int QS = TY == 12 ? 16 : 48;
+        gr_ld16(blk, 0, R);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gr_ld16(bg, QS + 32 * i, R + 4 + 4 * i);
+        if constexpr (TY == 13) gr_ld16(bg, 16, R + 20);
     }
-    return nullptr;
+}
+
+// Q6_K's scales and d, a step later (their registers then fit beside both super-blocks' codes).
+template <int TY>
+__device__ __forceinline__ void gr_load_scales(gr_ptr blk, uint32_t (&R)[gr_nraw<TY>()]) {
+    if constexpr (TY == 14) {
+        blk = (gr_ptr)((uint64_t)blk & ~3ull);
+        gr_ld16(blk, 192, R + 24);
+        R[28] = *reinterpret_cast<__attribute__((address_space(1))) const uint32_t*>(blk + 208);
+    }
+}
+
+// A loaded Q6_K super-block at ob (0 or 2) bytes into its dwords, moved to offset 0. The dword
+// after a lane's 16 bytes is the first one of the other lane half: its own chunk for g = 0, the
+// next one for g = 1 (v_permlane32_swap_b32: the upper half of one register for the lower of the other).
+template <int TY>
+__device__ __forceinline__ void gr_align(uint32_t (&R)[gr_nraw<TY>()], uint32_t ob, int g) {
+    if constexpr (TY == 14) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {  // chunk c + 1 still has its first dword
+            const auto sw = __builtin_amdgcn_permlane32_swap(R[4 * c], R[4 * c + 4], false, false);
+            const uint32_t nx = g ? sw[0] : sw[1];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) R[4 * c + d] = __builtin_amdgcn_alignbyte(d < 3 ? R[4 * c + d + 1] : nx, R[4 * c + d], ob);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) R[24 + d] = __builtin_amdgcn_alignbyte(R[25 + d], R[24 + d], ob);
+        R[28] >>= 8 * ob;
+    }
+}
+
+// Unit u's 16 values of this lane as 8 packed bf16 words: gf_decode_a's arithmetic, with every
+// shift and mask a constant and a dword of four codes masked once.
+template <int TY>
+__device__ __forceinline__ void gr_decode(const uint32_t (&R)[gr_nraw<TY>()], int u, int g, uint32_t (&o)[8]) {
+    if constexpr (TY == 14) {
+        const int t = u & 3;
+        const uint32_t sc = R[24 + (u >> 1)] >> (16 * (u & 1) + 8 * g);
+        const float dd = 0.25f * (f16_bits_to_f32(R[28] & 0xFFFFu) * (float)(int8_t)(sc & 0xFFu));
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const uint32_t ql = R[8 * (u >> 2) + 4 * (t & 1) + w], qh = R[16 + 4 * (u >> 2) + w];
+            // four signed bytes 4 (q - 32): q ^ 32 is q - 32 in 6-bit two's complement
+            uint32_t y = (((t >> 1 ? ql >> 2 : ql << 2) & 0x3C3C3C3Cu) | ((qh << (6 - 2 * t)) & 0xC0C0C0C0u)) ^ 0x80808080u;
+            asm("" : "+v"(y));
+            o[2 * w] = pack_bf16x2(dd * (float)(int8_t)(y & 0xFFu), dd * (float)(int8_t)((y >> 8) & 0xFFu));
+            o[2 * w + 1] = pack_bf16x2(dd * (float)(int8_t)((y >> 16) & 0xFFu), dd * (float)(int8_t)(y >> 24));
+        }
+    } else {
+        const uint32_t s3[3] = {R[1], R[2], R[3]};
+        uint32_t sc, m;
+        k_scale_min(s3, u, sc, m);
+        const float a = f16_bits_to_f32(R[0] & 0xFFFFu) * (float)sc, c = f16_bits_to_f32(R[0] >> 16) * (float)m;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            uint32_t q = (R[4 + 4 * (u >> 1) + w] >> (4 * (u & 1))) & 0x0F0F0F0Fu;
+            if constexpr (TY == 13) q |= (u < 4 ? R[20 + w] << (4 - u) : R[20 + w] >> (u - 4)) & 0x10101010u;
+            asm("" : "+v"(q));
+            o[2 * w] = pack_bf16x2(a * (float)(q & 0xFFu) - c, a * (float)((q >> 8) & 0xFFu) - c);
+            o[2 * w + 1] = pack_bf16x2(a * (float)((q >> 16) & 0xFFu) - c, a * (float)(q >> 24) - c);
+        }
+    }
+}
+
+// One tile with MT blocks of 32 sorted rows.
+template <int TY, bool GU, int MT>
+__device__ __forceinline__ void gr_tile(const GfGemm& p, const GfEntry& en, int n0, uint8_t* smem) {
+    constexpr int NR = gr_nraw<TY>(), NL = gr_nload<TY>(), TS = GfType<TY>::PB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), g = lane >> 5, rr = lane & 31;
+    const int K = p.K, KU = K / 32;
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
+
+    // This lane's weight row, every eighth from the wave's first: its place ph in its first
+    // super-block is the same for all rows of the wave (rows past the matrix read one of them).
+    int row = n0 + wave + 8 * (GU ? rr & 15 : rr);
+    if (row >= p.N) row = wave;
+    const int ph = uniform((int)(((uint32_t)row * (uint32_t)KU) & 7u));
+    const int nsb = (ph + KU + 7) >> 3;  // super-blocks of the row
+    const gr_ptr blk0 = (gr_ptr)(p.pool + (int64_t)en.slot * p.slot_bytes + (GU && rr >= 16 ? p.w2_off : p.w_off) +
+                                 (int64_t)TS * (((uint32_t)row * (uint32_t)KU) >> 3));
+    auto blk = [&](int q) { return blk0 + (uint32_t)(TS * (q < nsb ? q : nsb - 1)); };  // past the row: its last one
+
+    // Activation tiles: row r holds sorted row r's step as 16 chunks, chunk c in slot c ^ (r % 16);
+    // copy i of wave w fills rows 32 i + 4 w .. + 3 (lane l: row + l / 16, slot l % 16). Rows past
+    // the tile's and columns past K read zeros (an offset past the end).
+    const v4i_t rx = gf_desc(reinterpret_cast<const uint8_t*>(p.src), p.src_bytes);
+    uint32_t xo[MT];
+    const int xc = (lane & 15) ^ ((4 * wave + (lane >> 4)) & 15);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int r = 32 * i + 4 * wave + (lane >> 4);
+        xo[i] = 0x80000000u;
+        if (r < en.rows) {
+            const int a = GU ? p.perm[en.row0 + r] / p.k : en.row0 + r;
+            xo[i] = (uint32_t)((int64_t)a * K * 2) + 16u * (uint32_t)xc;
+        }
+    }
+    const int xsteps = (KU + 3) / 4;
+    auto issue_x = [&](int s) {
+        if (s >= xsteps) return;
+        const uint32_t t = lds0 + (uint32_t)(s % GR_RING) * GR_XB + (uint32_t)(4 * wave) * GR_RS;
+        const bool past = GR_KS * s + 8 * xc >= K;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            gf_dma(rx, past ? 0x80000000u : xo[i] + (uint32_t)s * GR_RS, t + (uint32_t)(32 * i) * GR_RS);
+    };
+
+    v16f_t acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+
+    // B operands: K step s2 of a unit covers its values 8 s2 .. + 7 (g = 0) and 16 + 8 s2 .. (g = 1)
+    const uint32_t xs = (uint32_t)(rr * GR_RS + 16 * ((2 * g) ^ (rr & 15)));
+    // units 4 h .. 4 h + 3 of super-block q: unit j of the row sits in step j / 4's tile
+    auto half = [&](const uint32_t (&R)[NR], int q, auto hc) {
+        constexpr int H = decltype(hc)::value;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = 8 * q + 4 * H + i - ph;
+            if (j < 0 || j >= KU) continue;  // wave-uniform: another row's
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t av[8];
+            gr_decode<TY>(R, 4 * H + i, g, av);
+            const uint32_t xa = (xs ^ (64u * (uint32_t)(j & 3))) + (uint32_t)((j >> 2) & 3) * GR_XB;
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+                const bf16x8 A = __builtin_bit_cast(bf16x8, u32x4{av[4 * s2], av[4 * s2 + 1], av[4 * s2 + 2], av[4 * s2 + 3]});
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const bf16x8 B = *reinterpret_cast<const bf16x8*>(smem + (xa ^ (16u * s2)) + 32 * t * GR_RS);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, acc[t], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    // Super-block q (steps 2 q and 2 q + 1) from C, the next one into F. Every wait is explicit as
+    // the compiler does not count the copies.
+    auto block = [&](int q, uint32_t (&C)[NR], uint32_t (&F)[NR]) {
+        // step 2 q: its activations and weights have landed, everywhere after the barrier; the tile
+        // that step 2 q + 1's activations take was last read before it
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NR; ++i) asm volatile("" : "+v"(C[i]));  // loaded: no later wait for them
+        __syncthreads();
+        issue_x(2 * q + 1);
+        gr_align<TY>(C, (uint32_t)(uint64_t)blk(q) & 3u, g);
+        __builtin_amdgcn_sched_barrier(0);  // F's registers are free until here
+        gr_load<TY>(blk(q + 1), g, F);
+        half(C, q, std::integral_constant<int, 0>{});
+        // step 2 q + 1: all but the newest loads, the next super-block's, have landed
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+        __syncthreads();
+        issue_x(2 * q + 2);
+        gr_load_scales<TY>(blk(q + 1), F);
+        half(C, q, std::integral_constant<int, 1>{});
+    };
+    const int blocks = (KU + 14) >> 3;  // of the rows that start last in their first one
+    uint32_t R0[NR], R1[NR];
+    gr_load<TY>(blk(0), g, R0);
+    gr_load_scales<TY>(blk(0), R0);
+    issue_x(0);
+    for (int q = 0; q < blocks; q += 2) {
+        block(q, R0, R1);
+        if (q + 1 < blocks) block(q + 1, R1, R0);
+    }
+
+    // Results into LDS as bf16 rows, then whole 16-byte pieces of them out. acc[t][4u + r] = the
+    // wave's weight row 8u + 4g + r (gate_up: rows 0 .. 15 gate, 16 .. 31 the same up rows),
+    // sorted row 32 t + rr.
+    constexpr int C = GU ? 128 : 256, SS = C + 8;  // columns, padded row
+    static_assert(GF_BM * SS * 2 <= GR_LDS, "staged results");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    uint16_t* stage = reinterpret_cast<uint16_t*>(smem);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        uint16_t* st = stage + (32 * t + rr) * SS + wave;
+#pragma unroll
+        for (int i = 0; i < (GU ? 8 : 16); ++i) {
+            const int c = 8 * (8 * (i >> 2) + 4 * g + (i & 3));
+            float v = acc[t][i];
+            if constexpr (GU) v = p.L.act == TSA_ACT_SWIGLU_OAI ? swiglu_oai_fast(p.L, v, acc[t][i + 8]) : silu_mul_fast(v, acc[t][i + 8]);
+            st[c] = f32_to_bf16_bits(v);
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < en.rows * (C / 8); i += GF_THREADS) {
+        const int r = i / (C / 8), c = 8 * (i % (C / 8));
+        if (n0 + c >= p.N) continue;
+        const int64_t orow = GU ? (int64_t)(en.row0 + r) : (int64_t)p.perm[en.row0 + r];
+        *reinterpret_cast<uint4*>(p.out + orow * p.N + n0 + c) = *reinterpret_cast<const uint4*>(stage + r * SS + c);
+    }
+}
+
+template <int TY, bool GU>
+__global__ void __launch_bounds__(GF_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) gf_reg_kernel(GfGemm p) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tiles = (int)gridDim.x, nact = *p.n_entries * tiles;
+    const int lin = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    if (lin >= nact) return;  // workgroup-uniform
+    const int xcd = lin & 7, q8 = nact >> 3, rem = nact & 7;
+    const int wid = xcd * q8 + (xcd < rem ? xcd : rem) + (lin >> 3);  // as gf_gemm_kernel
+    const int en_i = wid / tiles, tile = wid - en_i * tiles;
+    const GfEntry en = p.table[en_i];
+    const int n0 = tile * (GU ? GF_BN : 2 * GF_BN);
+    if (en.rows <= 32) gr_tile<TY, GU, 1>(p, en, n0, smem);
+    else gr_tile<TY, GU, 2>(p, en, n0, smem);
+}
+
+template <bool GU>
+const void* gr_pick(int t) {
+    return t == 12   ? reinterpret_cast<const void*>(&gf_reg_kernel<12, GU>)
+           : t == 13 ? reinterpret_cast<const void*>(&gf_reg_kernel<13, GU>)
+                     : reinterpret_cast<const void*>(&gf_reg_kernel<14, GU>);
 }
 
 template <int TY, bool GU>
@@ -651,10 +864,6 @@ const void* gf_step_pick(int t, bool gu) {
 }
 
 int gf_step_lds_of(int t) { return t == 12 ? gf_step_lds<12>() : t == 13 ? gf_step_lds<13>() : gf_step_lds<14>(); }
-
-int gf_lds_of(int t) {
-    return t == 8 ? gf_lds<8, false>() : t == 12 ? gf_lds<12, true>() : t == 13 ? gf_lds<13, true>() : gf_lds<14, true>();
-}
 
 int64_t gf_al256(int64_t v) { return (v + 255) / 256 * 256; }
 
@@ -722,17 +931,23 @@ int gf_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_slots,
     int rc = launch_group_kernel(idx, n, (int)E, counts, offsets, perm, stream, expert_slot, n_slots, GF_BM, nent, table);
     if (rc) return rc;
 
-    // a K-quant matrix whose K is a multiple of 256 takes gf_step_kernel; one whose K is not,
-    // the straddling variant of gf_gemm_kernel; Q8_0 its plain variant
-    const bool sd_gu = L.gate_type != 8 && L.hidden % GF_KP != 0, sd_dn = L.down_type != 8 && L.inter % GF_KP != 0;
-    const bool st_gu = L.gate_type != 8 && !sd_gu, st_dn = L.down_type != 8 && !sd_dn;
-    const void* f_gu = st_gu ? gf_step_pick(L.gate_type, true) : gf_pick(L.gate_type, true);
-    const void* f_dn = st_dn ? gf_step_pick(L.down_type, false) : gf_pick(L.down_type, false);
-    const int lds_gu = st_gu ? gf_step_lds_of(L.gate_type) : gf_lds_of(L.gate_type),
-              lds_dn = st_dn ? gf_step_lds_of(L.down_type) : gf_lds_of(L.down_type);
-    for (auto [f, b] : {std::pair<const void*, int>{f_gu, lds_gu}, std::pair<const void*, int>{f_dn, lds_dn}}) {
-        const hipError_t e = ensure_dynamic_lds(f, b);
-        TSA_REQUIRE(e == hipSuccess, TSA_ERR_HIP, "hipFuncSetAttribute(LDS %d): %s", b, hipGetErrorString(e));
+    // Q8_0 takes gf_gemm_kernel; a K-quant matrix gf_step_kernel where its rows start with a
+    // super-block (K % 256 == 0), else gf_reg_kernel (on aligned rows the two measure alike)
+    struct Pick {
+        const void* fn;
+        int lds, cols;  // output columns per tile
+    };
+    auto pick = [](int t, int64_t K, bool gu) -> Pick {
+        if (t == 8)
+            return {gu ? reinterpret_cast<const void*>(&gf_gemm_kernel<true>) : reinterpret_cast<const void*>(&gf_gemm_kernel<false>),
+                    GF_LDS, gu ? GF_BN / 2 : GF_BN};
+        if (K % GF_KP == 0) return {gf_step_pick(t, gu), gf_step_lds_of(t), gu ? GF_BN / 2 : GF_BN};
+        return {gu ? gr_pick<true>(t) : gr_pick<false>(t), GR_LDS, gu ? GF_BN : 2 * GF_BN};
+    };
+    const Pick gu = pick(L.gate_type, L.hidden, true), dn = pick(L.down_type, L.inter, false);
+    for (const Pick& f : {gu, dn}) {
+        const hipError_t e = ensure_dynamic_lds(f.fn, f.lds);
+        TSA_REQUIRE(e == hipSuccess, TSA_ERR_HIP, "hipFuncSetAttribute(LDS %d): %s", f.lds, hipGetErrorString(e));
     }
     const unsigned max_entries = (unsigned)(n / GF_BM + (E < n ? E : n) + 1);
     auto mat_bytes = [](int t, int64_t rows, int64_t K) {  // rows K values as one run of blocks
@@ -757,8 +972,8 @@ int gf_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_slots,
     g.w2_off = L.up_off;
     g.w_bytes = mat_bytes(L.gate_type, I, H);
     void* args[] = {&g};
-    TSA_HIP_CHECK(hipLaunchKernel(f_gu, dim3((unsigned)((I + GF_BN / 2 - 1) / (GF_BN / 2)), max_entries),
-                                  dim3(GF_THREADS), args, lds_gu, stream));
+    TSA_HIP_CHECK(hipLaunchKernel(gu.fn, dim3((unsigned)((I + gu.cols - 1) / gu.cols), max_entries),
+                                  dim3(GF_THREADS), args, gu.lds, stream));
     // down: h [n, I] -> yk [n, H] by assignment id
     g.src = h;
     g.src_bytes = n * L.inter * 2;
@@ -768,8 +983,8 @@ int gf_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_slots,
     g.w_off = L.down_off;
     g.w2_off = L.down_off;
     g.w_bytes = mat_bytes(L.down_type, H, I);
-    TSA_HIP_CHECK(hipLaunchKernel(f_dn, dim3((unsigned)((H + GF_BN - 1) / GF_BN), max_entries),
-                                  dim3(GF_THREADS), args, lds_dn, stream));
+    TSA_HIP_CHECK(hipLaunchKernel(dn.fn, dim3((unsigned)((H + dn.cols - 1) / dn.cols), max_entries),
+                                  dim3(GF_THREADS), args, dn.lds, stream));
     return pf_combine(yk, idx, weights, expert_slot, E, n_slots, T, k, H, y, y_dtype, stream);
 }
 
