@@ -69,6 +69,19 @@ def test_prefill_more_tiles_than_workgroups(H, I, T):
     assert_close_bf16(y, _ref(experts, synth.bf16_to_f32(x_bits), idx, w), f"prefill H={H} I={I} T={T}")
 
 
+@pytest.mark.parametrize("E,T,mfma", [(1, 70, _lib.PREFILL_FP6), (334, 24, _lib.PREFILL_BF16), (336, 700, _lib.PREFILL_FP6)])
+def test_prefill_preparation_by_expert_count(E, T, mfma):
+    """One expert; the most experts that 16 waves group within 64 KB of LDS (334), and more
+    (8 waves); in rows of several batches of 64 per wave, and without records to form."""
+    H, I, k = 64, 32, min(E, 4)
+    rng, L, experts, pool = _pool(H, I, E, seed=E, mfma=mfma)
+    x_bits = synth.bf16_normal(rng, (T, H))
+    idx, w = oex.route_topk_then_softmax(synth.zipf_logits(rng, T, E), k)
+    y = ops.moe_prefill(L, pool, torch.arange(E, dtype=torch.int32, device="cuda"),
+                        torch.from_numpy(idx.astype(np.int32)).cuda(), torch.from_numpy(w).cuda(), bf16_dev(x_bits))
+    assert_close_bf16(y, _ref(experts, synth.bf16_to_f32(x_bits), idx, w), f"prefill E={E} T={T}")
+
+
 def test_prefill_only_full_row_tiles():
     """Every expert gets exactly 128 or 256 rows: the tile table holds full entries only."""
     H, I, E, k, T = 512, 256, 5, 2, 384

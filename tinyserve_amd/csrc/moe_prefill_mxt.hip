@@ -1,9 +1,9 @@
 // Batched (prefill) MoE over MXFP4 experts in the 16-row MFMA tile order: the grouped
 // expert GEMMs on the matrix cores.
 //
-// After the (token, expert) assignments are sorted expert-major (group_kernel), each
+// After the (token, expert) assignments are sorted expert-major (group_assignments), each
 // expert's rows form one contiguous run of the sorted order, cut into tiles of up to 128
-// rows (pf_table_kernel). Two persistent GEMM launches then cover every (row tile, weight
+// rows (pf_table). Two persistent GEMM launches then cover every (row tile, weight
 // tile) pair:
 //   gate_up: h[i, :] = SwiGLU(x[token(i)] W_gu^T + b_gu), bf16, in sorted order;
 //   down:    yk[a, :] = h[i] W_dn^T + b_dn, bf16, by assignment id a = perm[i]
@@ -33,6 +33,7 @@
 
 #include "fused_common.h"
 #include "mfma_tile.h"
+#include "moe_group.h"
 #include "fp6_terms.h"
 
 namespace tsa {
@@ -910,12 +911,12 @@ __global__ void __launch_bounds__(PF_THREADS) pf6_gemm_kernel(PfGemm p) {
 // row tiles stay on few XCDs and share its weights in L2; then the partial ones, largest
 // first, each go to the group with the least estimated cost so far (PF_COST0 + rows per
 // entry). Within a group the full entries come first, then the partial ones largest first. Equal-row partial entries are ranked in any order: the results do not
-// depend on the order. Also zeroes the GEMMs' tile counters. E <= 1024.
-__global__ void __launch_bounds__(1024) pf_table_kernel(const int32_t* __restrict__ counts,
-                                                        const int32_t* __restrict__ offsets,
-                                                        const int32_t* __restrict__ expert_slot, int E,
-                                                        int64_t n_slots, int* __restrict__ n_entries,
-                                                        PfEntry* __restrict__ table, int* __restrict__ ctr) {
+// depend on the order. Also zeroes the GEMMs' tile counters. 1024 threads, E <= 1024; cnt: E
+// ints of LDS.
+__device__ __forceinline__ void pf_table(const int32_t* __restrict__ idx, int64_t n,
+                                         const int32_t* __restrict__ expert_slot, int E, int64_t n_slots,
+                                         int* __restrict__ n_entries, PfEntry* __restrict__ table,
+                                         int* __restrict__ ctr, int* cnt) {
     __shared__ int wsum[16];
     __shared__ int hist[PF_BM];    // partial entries with r rows
     __shared__ int pos[PF_BM];     // rank (offset by the full entries) of the next partial entry with r rows
@@ -925,16 +926,28 @@ __global__ void __launch_bounds__(1024) pf_table_kernel(const int32_t* __restric
     const int e = threadIdx.x;
     if (e < PF_CTR_INTS) ctr[e] = 0;
     if (e < PF_BM) hist[e] = 0;
-    int slot = -1, c = 0, nt = 0, r = 0, o = 0;
-    if (e < E) {  // the three loads go out together
+    int slot = -1, c = 0, nt = 0, r = 0;
+    if (e < E) {
+        cnt[e] = 0;
         slot = expert_slot[e];
-        c = counts[e];
-        o = offsets[e];
-        if (slot >= 0 && slot < n_slots) {
-            nt = c / PF_BM;
-            r = c % PF_BM;
-        }
     }
+    __syncthreads();
+    for (int64_t a0 = e; a0 < n; a0 += 1024 * GROUP_AHEAD) {  // the experts' counts
+        int ev[GROUP_AHEAD];
+#pragma unroll
+        for (int j = 0; j < GROUP_AHEAD; ++j) ev[j] = a0 + 1024 * j < n ? idx[a0 + 1024 * j] : -1;
+#pragma unroll
+        for (int j = 0; j < GROUP_AHEAD; ++j)
+            if (ev[j] >= 0 && ev[j] < E) atomicAdd(&cnt[ev[j]], 1);
+    }
+    __syncthreads();
+    if (e < E) c = cnt[e];
+    if (slot >= 0 && slot < n_slots) {
+        nt = c / PF_BM;
+        r = c % PF_BM;
+    }
+    int all_rows;
+    const int o = block_incl_sum(c, wsum, all_rows) - c;  // the expert's first sorted row
     __syncthreads();  // hist cleared
     if (r > 0) atomicAdd(&hist[r], 1);
     int F;
@@ -1011,9 +1024,8 @@ __global__ void __launch_bounds__(1024) pf_table_kernel(const int32_t* __restric
 
 // x [rows, K] bf16 -> fp6 records (rows of MP records; blocks at or past K as zero codes with a
 // unit scale). One thread per (row, 32-value block).
-__global__ void __launch_bounds__(256) pf_quant_kernel(const uint16_t* __restrict__ x, int64_t rows, int K, int MP,
-                                                       uint8_t* __restrict__ out) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pf_quant(const uint16_t* __restrict__ x, int64_t rows, int K, int MP,
+                                         uint8_t* __restrict__ out, int64_t g) {
     const int nb = 4 * MP;
     if (g >= rows * nb) return;
     const int64_t r = g / nb;
@@ -1045,6 +1057,35 @@ __global__ void __launch_bounds__(256) pf_quant_kernel(const uint16_t* __restric
     *reinterpret_cast<uint4*>(rec + 48 * bq + 16) = make_uint4(hi[4], hi[5], lo[0], lo[1]);
     *reinterpret_cast<uint4*>(rec + 48 * bq + 32) = make_uint4(lo[2], lo[3], lo[4], lo[5]);
     rec[PF_QSCALE + bq] = (uint8_t)sc;
+}
+
+// All that the GEMMs need before them, in one launch: workgroup 0 groups the assignments
+// (perm), workgroup 1 counts them by itself and forms the tile table, the rest form x's fp6
+// records. Each was a launch of its own, small ones mostly launch: 32 experts, hidden 2880, top
+// 4, us: 24 tokens 4.2 + 5.5 + 4.2 -> 6.5 (and two launch gaps), 2047 tokens 8.1 + 9.0 + 7.7 -> 13.
+struct PfPrep {
+    const int32_t* idx;
+    int64_t n;
+    int E, nw;                // nw: waves that group
+    int32_t *counts, *offsets, *perm;
+    const int32_t* expert_slot;
+    int64_t n_slots;
+    int* n_entries;
+    PfEntry* table;
+    int* ctr;
+    const uint16_t* x;
+    int64_t T;
+    int K, MP;
+    uint8_t* xq;
+};
+__global__ void __launch_bounds__(1024) pf_prepare_kernel(PfPrep p) {
+    extern __shared__ __align__(16) unsigned char gsm[];
+    if (blockIdx.x == 0)
+        group_assignments<false>(p.idx, p.n, p.E, p.counts, p.offsets, p.perm, GroupTiles{}, p.nw, gsm);
+    else if (blockIdx.x == 1)
+        pf_table(p.idx, p.n, p.expert_slot, p.E, p.n_slots, p.n_entries, p.table, p.ctr, reinterpret_cast<int*>(gsm));
+    else
+        pf_quant(p.x, p.T, p.K, p.MP, p.xq, (int64_t)(blockIdx.x - 2) * 1024 + threadIdx.x);
 }
 
 // y[t] = sum_j w[t, j] yk[t k + j] over the live assignments, j in order; 8 columns per thread.
@@ -1149,10 +1190,6 @@ int64_t pf_mxt_workspace_bytes(const tsa_expert_layout& L, int64_t T, int k, int
     return pf_ws_layout(L, T, k, E).total;
 }
 
-int launch_group_kernel(const int32_t* idx, int64_t n, int E, int32_t* counts, int32_t* offsets, int32_t* perm,
-                        hipStream_t stream, const int32_t* expert_slot = nullptr, int64_t n_slots = 0,
-                        int tile_rows = 0, int* n_entries = nullptr, void* table = nullptr);
-
 // y[t] = sum_j w[t, j] yk[t k + j] over the live assignments, j in order (H % 8 == 0).
 int pf_combine(const uint16_t* yk, const int32_t* idx, const float* w, const int32_t* expert_slot, int64_t E,
                int64_t n_slots, int64_t T, int k, int H, void* y, int y_dtype, hipStream_t stream) {
@@ -1177,13 +1214,18 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
     uint16_t* yk = reinterpret_cast<uint16_t*>(ws + w.yk);
     const int H = (int)L.hidden, I = (int)L.inter;
 
-    int rc = launch_group_kernel(idx, T * k, (int)E, counts, offsets, perm, stream);
-    if (rc) return rc;
-    hipLaunchKernelGGL(pf_table_kernel, dim3(1), dim3(1024), 0, stream, counts, offsets, expert_slot, (int)E, n_slots,
-                       nent, table, ctr);
+    const bool q6 = L.prefill_mfma == TSA_PREFILL_FP6;
+    uint8_t* xq = ws + w.xq;
+    const int MPH = (H + 127) / 128;
+    // 16 waves group where their LDS leaves the records' workgroups two per CU, else 8
+    const int nw = group_lds_bytes((int)E, 16) <= 64 * 1024 ? 16 : 8, glds = group_lds_bytes((int)E, nw);
+    const hipError_t le = ensure_dynamic_lds(reinterpret_cast<const void*>(pf_prepare_kernel), glds);
+    TSA_REQUIRE(le == hipSuccess, TSA_ERR_HIP, "hipFuncSetAttribute(LDS %d): %s", glds, hipGetErrorString(le));
+    const PfPrep pp{idx, T * k, (int)E, nw, counts, offsets, perm, expert_slot, n_slots, nent, table, ctr, x, T, H, MPH, xq};
+    const int64_t recs = q6 ? T * 4 * MPH : 0;
+    hipLaunchKernelGGL(pf_prepare_kernel, dim3((unsigned)(2 + (recs + 1023) / 1024)), dim3(1024), glds, stream, pp);
     TSA_LAUNCH_CHECK();
 
-    const bool q6 = L.prefill_mfma == TSA_PREFILL_FP6;
     const void* f_gu = q6 ? reinterpret_cast<const void*>(pf6_gemm_kernel<true>) : reinterpret_cast<const void*>(pf_gemm_kernel<true>);
     const void* f_dn = q6 ? reinterpret_cast<const void*>(pf6_gemm_kernel<false>) : reinterpret_cast<const void*>(pf_gemm_kernel<false>);
     const int lds = q6 ? P6_LDS : PF_LDS;
@@ -1201,13 +1243,6 @@ int pf_mxt_prefill(const tsa_expert_layout& L, const uint8_t* pool, int64_t n_sl
     g.ctr = ctr;
     g.k = k;
     void* args[] = {&g};
-    uint8_t* xq = ws + w.xq;
-    if (q6) {  // x as fp6 records
-        const int64_t threads = T * 4 * ((H + 127) / 128);
-        hipLaunchKernelGGL(pf_quant_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, x, T, H,
-                           (H + 127) / 128, xq);
-        TSA_LAUNCH_CHECK();
-    }
     // gate_up: [2I, H] -> h
     g.src = q6 ? static_cast<const void*>(xq) : static_cast<const void*>(x);
     g.src_rows = T;
