@@ -128,11 +128,17 @@ def stream_handle(device: torch.device | None = None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def tensor_stream(t: torch.Tensor) -> int:
+    """The current stream of a GPU tensor's device, as stream_handle gives it, without the
+    ``torch.cuda.Stream`` object around it (over 1 us of a 9 us call)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
 def require_device(*tensors: torch.Tensor, what: str = "tensor") -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"{what} must be on CUDA")

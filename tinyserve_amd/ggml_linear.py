@@ -50,12 +50,14 @@ class GGMLLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not _check_ggml():
             raise RuntimeError("GGMLLinear needs the tinyserve_amd HIP library (build it with __graft_entry__.build())")
-        lead = x.shape[:-1]
-        out = ops.gguf_matvec(x.reshape(-1, self.in_features), self._qweight, self._ggml_type, self.out_features,
-                              self.in_features, out_dtype=x.dtype)
-        if self.bias is not None:
-            out = out + self.bias
-        return out.reshape(*lead, self.out_features)
+        K = self.in_features
+        rows = x.dim() == 2 and x.shape[1] == K > 0  # already rows: no views to make
+        out = ops.gguf_matvec(x if rows else x.reshape(-1, K), self._qweight, self._ggml_type, self.out_features, K,
+                              out_dtype=x.dtype)
+        bias = self.bias
+        if bias is not None:
+            out = out + bias
+        return out if rows else out.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self) -> str:
         names = {8: "Q8_0", 12: "Q4_K", 13: "Q5_K", 14: "Q6_K"}

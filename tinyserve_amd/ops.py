@@ -13,8 +13,14 @@ import torch
 from . import _lib
 
 
-def _stream(t: torch.Tensor) -> int:
-    return _lib.stream_handle(t.device)
+_stream = _lib.tensor_stream
+
+
+def _rows(x: torch.Tensor, K: int) -> torch.Tensor:
+    """x as contiguous rows of K values (a [T, K] x as it is: no view to make)."""
+    if x.dim() == 2 and x.shape[1] == K > 0:
+        return x.contiguous()
+    return x.reshape(-1, K).contiguous()
 
 
 # ----------------------------------------------------------------------------- GGUF
@@ -48,10 +54,9 @@ def gguf_matvec(x: torch.Tensor, w: torch.Tensor, ggml_type: int, out_features: 
     if w.dtype != torch.uint8:
         raise RuntimeError("weight_data must be uint8")
     K, N = int(in_features), int(out_features)
-    x2 = x.reshape(-1, K) if x.numel() % K == 0 else x.reshape(1, -1)
-    x2 = x2.contiguous()
+    x2 = _rows(x, K) if x.numel() % K == 0 else x.reshape(1, -1).contiguous()
     T = x2.shape[0]
-    y = torch.empty((T, N), dtype=out_dtype or x.dtype, device=x.device)
+    y = x.new_empty((T, N), dtype=out_dtype or x.dtype)
     w = w.contiguous()
     _lib.check(_lib.load().tsa_gguf_matvec(int(ggml_type), w.data_ptr(), w.numel(), x2.data_ptr(),
                                            _lib.tsa_dtype(x2.dtype), T, K, y.data_ptr(), _lib.tsa_dtype(y.dtype), N,
@@ -111,9 +116,9 @@ def mxfp4_matvec(x: torch.Tensor, blocks: torch.Tensor, scales: torch.Tensor, bi
     _lib.require_device(x, blocks, scales, what="tensor")
     N = blocks.shape[0]
     K = blocks[0].numel() * 2
-    x2 = x.reshape(-1, K).contiguous()
+    x2 = _rows(x, K)
     T = x2.shape[0]
-    y = torch.empty((T, N), dtype=out_dtype or x.dtype, device=x.device)
+    y = x.new_empty((T, N), dtype=out_dtype or x.dtype)
     blocks, scales = blocks.contiguous(), scales.contiguous()
     b = None if bias is None else bias.contiguous()
     _lib.check(_lib.load().tsa_mxfp4_matvec(blocks.data_ptr(), scales.data_ptr(), _lib.ptr(b),
@@ -134,7 +139,7 @@ ROUTE_MODES = {
 def route_topk(logits: torch.Tensor, top_k: int, mode: str = "topk_then_softmax") -> tuple[torch.Tensor, torch.Tensor]:
     """(idx int32 [T, k], weights float32 [T, k]) from router logits [T, E]."""
     _lib.require_device(logits, what="logits")
-    lg = logits.reshape(-1, logits.shape[-1]).contiguous()
+    lg = _rows(logits, logits.shape[-1])
     T, E = lg.shape
     idx = torch.empty((T, top_k), dtype=torch.int32, device=lg.device)
     w = torch.empty((T, top_k), dtype=torch.float32, device=lg.device)
@@ -150,10 +155,10 @@ def router_logits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
     ``F.linear`` returns it)."""
     _lib.require_device(x, weight, *([bias] if bias is not None else []), what="tensor")
     E, H = weight.shape
-    x2 = x.reshape(-1, H).contiguous()
+    x2 = _rows(x, H)
     w = weight.contiguous()
     b = bias.contiguous() if bias is not None else None
-    out = torch.empty((x2.shape[0], E), dtype=out_dtype or weight.dtype, device=x.device)
+    out = x.new_empty((x2.shape[0], E), dtype=out_dtype or weight.dtype)
     _lib.check(_lib.load().tsa_router_logits(
         x2.data_ptr(), _lib.tsa_dtype(x2.dtype), x2.shape[0], H, w.data_ptr(), _lib.tsa_dtype(w.dtype), _lib.ptr(b),
         _lib.tsa_dtype(b.dtype) if b is not None else 0, E, out.data_ptr(), _lib.tsa_dtype(out.dtype), _stream(x)))
