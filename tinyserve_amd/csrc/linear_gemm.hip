@@ -212,6 +212,9 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
             for (int w = 0; w < 4; ++w) {
                 uint32_t q = (qs[w] >> sh) & 0x0F0F0F0Fu;
                 if constexpr (F == 13) q |= ((qh[w] >> u) & 0x01010101u) << 4;
+                // masked once for its four bytes (the compiler extracts each by itself otherwise:
+                // Q4_K 4096 x 2048, 512 tokens, 27.3 -> 24.4 us per call)
+                asm("" : "+v"(q));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[4 * w + e] = a * (float)((q >> (8 * e)) & 0xFFu) - c;
             }
@@ -237,7 +240,8 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 // four signed bytes 4 (q - 32): q ^ 32 is q - 32 in 6-bit two's complement
-                const uint32_t q = ((((ql[w] >> shl) & 0x0F0F0F0Fu) | (((qh[w] >> shh) & 0x03030303u) << 4)) ^ 0x20202020u) << 2;
+                uint32_t q = ((((ql[w] >> shl) & 0x0F0F0F0Fu) | (((qh[w] >> shh) & 0x03030303u) << 4)) ^ 0x20202020u) << 2;
+                asm("" : "+v"(q));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[4 * w + e] = dd * (float)(int8_t)((q >> (8 * e)) & 0xFFu);
             }
