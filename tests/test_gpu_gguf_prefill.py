@@ -215,9 +215,10 @@ def test_gguf_grouped_prefill_straddling_rows(types, H, I, pad):
     assert_close_bf16(y, ref, f"GGUF grouped prefill, straddling rows, types {types}, H {H}, I {I}")
 
 
-@pytest.mark.parametrize("types,H,I,pad", [((12, 12, 12), 64, 32, 0), ((14, 14, 14), 96, 32, 6), ((13, 13, 14), 800, 384, 0)])
-def test_gguf_grouped_prefill_straddling_rows_tile_edges(types, H, I, pad):
-    """Straddling rows of 1, 2, 3, 12 and 25 units (a row inside one super-block, or over up to
+@pytest.mark.parametrize("types,H,I,pad", [((12, 12, 12), 64, 32, 0), ((14, 14, 14), 96, 32, 6), ((13, 13, 14), 800, 384, 0),
+                                           ((12, 12, 14), 512, 256, 0)])
+def test_gguf_grouped_prefill_tile_edges(types, H, I, pad):
+    """Aligned rows, and straddling rows of 1, 2, 3, 12 and 25 units (a row inside one super-block, or over up to
     five), weight rows that leave a tile part empty, and experts with 1, 32, 33, 64 and 65
     sorted rows (one or two blocks of 32, a second tile)."""
     rng = np.random.default_rng(500 + H + I + pad)
@@ -225,7 +226,7 @@ def test_gguf_grouped_prefill_straddling_rows_tile_edges(types, H, I, pad):
     idx = rng.permutation(np.repeat(np.arange(len(loads)), loads))[:, None]
     L, experts, pool = _pool(rng, H, I, types, len(loads), pad=pad)
     y, ref = _run(L, experts, pool, rng, len(idx), 1, len(loads), idx=idx, grouped=True)
-    assert_close_bf16(y, ref, f"GGUF grouped prefill, straddling tile edges, types {types}, H {H}, I {I}")
+    assert_close_bf16(y, ref, f"GGUF grouped prefill, tile edges, types {types}, H {H}, I {I}")
 
 
 def test_gguf_grouped_prefill_2880_wide_512_tokens():

@@ -453,6 +453,9 @@ template <int TY> __device__ __forceinline__ int gf_half_chunk(int c, int h) {
 // is half s % 2 of piece s / 2; wave kh decodes units 4 h + 2 kh and 4 h + 2 kh + 1 of it, and
 // the steps of a piece are unrolled and the two kh branches written out, so every unit index
 // and shift is a constant and the LDS addresses of the B operands and windows are fixed per lane.
+// A tile of at most 32 sorted rows neither copies nor multiplies the other 32 (Zipf top-8 of 128
+// experts, Q5_K gate_up / Q6_K down: 1024 tokens 148 + 106 -> 141 + 102 us, 300 tokens 84 + 57
+// -> 78 + 54, where HBM bounds it, 100 tokens, unchanged).
 template <int TY, bool GU>
 __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -509,11 +512,13 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
         rc0[i] = 16u * (uint32_t)gf_half_chunk<TY>(c, 0);
         rc1[i] = 16u * (uint32_t)gf_half_chunk<TY>(c, 1);
     }
+    const bool half = uniform(en.rows) <= 32;  // no sorted rows 32 .. 63: neither copied nor multiplied
     auto issue = [&](int s) {  // step s's activations and half windows, into tile and area s % 2
         const int pc = s >> 1, h = s & 1;
         const uint32_t t = lds0 + (uint32_t)h * GF_SXB + (uint32_t)(8 * wave) * GF_SRS;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) gf_dma(rx, xo[i] + (uint32_t)s * (2 * GF_KS), t + (uint32_t)(4 * i) * GF_SRS);
+        for (int i = 0; i < 2; ++i)
+            if (wave < 4 || !half) gf_dma(rx, xo[i] + (uint32_t)s * (2 * GF_KS), t + (uint32_t)(4 * i) * GF_SRS);
         const uint32_t ra = lds0 + GF_SROFF + (uint32_t)h * RAW;
 #pragma unroll
         for (int i = 0; i < RI; ++i) {
@@ -543,7 +548,7 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
 
     // units 4 h + 2 khc + uu of the step in tile / area h: each decoded straight into the A
     // operands of its two K steps, each times sorted rows 0 .. 31 and 32 .. 63
-    auto units = [&](const uint8_t* sb, int h, int khc) {
+    auto units = [&](const uint8_t* sb, int h, int khc, auto mt) {
 #pragma unroll
         for (int uu = 0; uu < 2; ++uu) {
             uint32_t av[8];
@@ -552,7 +557,7 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
             for (int s2 = 0; s2 < 2; ++s2) {
                 const bf16x8 A = __builtin_bit_cast(bf16x8, u32x4{av[4 * s2], av[4 * s2 + 1], av[4 * s2 + 2], av[4 * s2 + 3]});
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
+                for (int t = 0; t < decltype(mt)::value; ++t) {
                     const bf16x8 B = *reinterpret_cast<const bf16x8*>(xa[2 * uu + s2] + h * GF_SXB + 32 * t * GF_SRS);
                     acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, acc[t], 0, 0, 0);
                 }
@@ -564,17 +569,21 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
     // the barrier: every wave's copies of step s have landed and tile / area (s + 1) % 2, last
     // read in step s - 1, is free for step s + 1's copies.
     issue(0);
-    for (int pc = 0; pc < P; ++pc) {
-        const uint8_t* sbp = win + ((dg + (uint32_t)pc * PB) & WA);  // the block's place in its window
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            if (h == 0 || pc + 1 < P) issue(2 * pc + h + 1);
-            if (kh == 0) units(sbp + h * RAW, h, 0);
-            else units(sbp + h * RAW, h, 1);
+    auto run = [&](auto mt) {
+        for (int pc = 0; pc < P; ++pc) {
+            const uint8_t* sbp = win + ((dg + (uint32_t)pc * PB) & WA);  // the block's place in its window
+    #pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                if (h == 0 || pc + 1 < P) issue(2 * pc + h + 1);
+                if (kh == 0) units(sbp + h * RAW, h, 0, mt);
+                else units(sbp + h * RAW, h, 1, mt);
+            }
         }
-    }
+    };
+    if (half) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
     gf_store_tile<GU>(p, en, n0, acc, smem);
 }
 
