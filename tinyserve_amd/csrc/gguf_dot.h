@@ -191,7 +191,7 @@ __device__ __forceinline__ void gq_stage_raw(const uint8_t* base, uint32_t recor
     for (uint32_t c = 0; c < n; c += 1024) {
         const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst + c);
         if (c + 16 * lane < n)
-            asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(a0 + c + 16 * lane), "s"(r),
+            asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(a0 + c + 16 * lane), "s"(r),
                          "s"(m0)
                          : "memory", "m0");
     }
@@ -206,7 +206,7 @@ __device__ __forceinline__ void gq_stage_vec_raw(const uint8_t* base, uint32_t r
     for (uint32_t c = 0; c < n; c += 256) {
         const uint32_t m0 = __builtin_amdgcn_readfirstlane(dst + c + 16 * (c >> 8));
         if (lane < 16 && c + 16 * lane < n)
-            asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(a0 + c + 16 * lane), "s"(r),
+            asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(a0 + c + 16 * lane), "s"(r),
                          "s"(m0)
                          : "memory", "m0");
     }

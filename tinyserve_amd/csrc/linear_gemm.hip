@@ -55,7 +55,7 @@ __device__ __forceinline__ lg_v4i lg_desc(const void* p, uint32_t bytes) {
 // Lane l's 16 bytes at buffer offset voff land at LDS byte lds + 16 l (inline assembly: the
 // compiler would otherwise wait for every copy before any later LDS read).
 __device__ __forceinline__ void lg_dma(const lg_v4i& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r),
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r),
                  "s"(__builtin_amdgcn_readfirstlane((int)lds))
                  : "memory", "m0");
 }

@@ -593,11 +593,11 @@ __device__ bool wait_token(const MxtParams& p, int t, uint32_t want, int lane, i
 // lds + 16 lane (one 1 KB wave transfer); 4 bytes per lane (256 B) for the dword form.
 // Issued from inline assembly: the caller waits for them with its own s_waitcnt.
 __device__ __forceinline__ void lds_dma16_agent(const __amdgpu_buffer_rsrc_t& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen sc1 lds" ::"v"(voff), "s"(r), "s"(lds)
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen sc1 lds" ::"v"(voff), "s"(r), "s"(lds)
                  : "memory", "m0");
 }
 __device__ __forceinline__ void lds_dma4_agent(const __amdgpu_buffer_rsrc_t& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dword %0, %1, 0 offen sc1 lds" ::"v"(voff), "s"(r), "s"(lds)
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dword %0, %1, 0 offen sc1 lds" ::"v"(voff), "s"(r), "s"(lds)
                  : "memory", "m0");
 }
 

@@ -99,7 +99,7 @@ struct GfGemm {
 // One 1 KB copy: lane l's 16 bytes at buffer offset voff land at LDS byte lds + 16 l (the LDS
 // address is the wave's, taken from the first lane).
 __device__ __forceinline__ void gf_dma(const v4i_t& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r),
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r),
                  "s"(__builtin_amdgcn_readfirstlane((int)lds))
                  : "memory", "m0");
 }

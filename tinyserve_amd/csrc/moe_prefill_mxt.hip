@@ -113,11 +113,11 @@ __device__ __forceinline__ v4i buf_desc(const void* p, uint32_t bytes) {
 // waits for exactly what it needs (pf_wait). Loads return in order, so the compiler's own
 // waits for its loads can only get stricter, never too weak.
 __device__ __forceinline__ void pf_dma(const v4i& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds)
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds)
                  : "memory", "m0");
 }
 __device__ __forceinline__ void pf_dma4(const v4i& r, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds)
+    asm volatile("s_mov_b32 m0, %2\n\t" TSA_COPY_WAIT "buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds)
                  : "memory", "m0");
 }
 
@@ -431,13 +431,13 @@ constexpr int P6_STREAM = 8;  // rows of at least this many pieces run on into t
 // pf_dma / pf_dma4 to lds + IMM, with a scalar byte offset soff added to voff.
 template <int IMM>
 __device__ __forceinline__ void p6_dma(const v4i& r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
+    asm volatile("s_add_u32 m0, %3, %4\n\t" TSA_COPY_WAIT "buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
                  "s"(__builtin_amdgcn_readfirstlane((int)lds)), "n"(IMM)
                  : "memory", "m0", "scc");
 }
 template <int IMM>
 __device__ __forceinline__ void p6_dma4(const v4i& r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
+    asm volatile("s_add_u32 m0, %3, %4\n\t" TSA_COPY_WAIT "buffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
                  "s"(__builtin_amdgcn_readfirstlane((int)lds)), "n"(IMM)
                  : "memory", "m0", "scc");
 }

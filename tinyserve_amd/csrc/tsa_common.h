@@ -71,6 +71,14 @@ uint32_t mxt_wait_limit();
 
 
 // ---------------------------------------------------------------- device helpers
+// Wait states inside a copy to LDS that is written in inline assembly ("write m0" TSA_COPY_WAIT
+// "buffer_load .. lds"), where the compiler's hazard pass cannot put them: gfx950 wants one between
+// a scalar write of M0 and the copy that takes its LDS address from it, and five between a VALU
+// write of a scalar register (v_readfirstlane, or the v_readlane that reloads a spilled one) and the
+// copy that reads it as descriptor or offset. The M0 write and these four make the five. (One instead
+// of four, where no VALU write is near, measures the same: within 0.3% on every path.)
+#define TSA_COPY_WAIT "s_nop 3\n\t"
+
 // IEEE binary16 bits -> float by v_cvt_f32_f16: exact for every half, subnormals included
 // (HIP kernels run with f16/f64 denormals preserved; a signalling NaN comes back quiet).
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
