@@ -22,12 +22,12 @@ def _x(rng, T, K):
 
 def _check(y, x, w, bias=None):
     """Each result within one bf16 rounding (2^-9, twice that for a rounding on the edge) plus
-    the split weights' 2^-17 and fp32 summation (K 2^-24) of the sum of absolute products."""
+    fp32 summation (K 2^-24) of the sum of absolute products."""
     ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
     if bias is not None:
         ref, mag = ref + bias, mag + np.abs(bias)
     d = np.abs(y.double().cpu().numpy() - ref)
-    bound = 2.0 ** -8 * np.abs(ref) + (2.0 ** -17 + w.shape[1] * 2.0 ** -24) * mag
+    bound = 2.0 ** -8 * np.abs(ref) + w.shape[1] * 2.0 ** -24 * mag
     assert (d <= bound).all(), f"worst {np.max(d / np.maximum(bound, 1e-30)):.3f} of the bound"
 
 
@@ -111,3 +111,35 @@ def test_not_finite(fmt):
         assert np.array_equal(np.isnan(y[t]), np.isnan(ref[t])) and np.array_equal(y[t][np.isinf(ref[t])], ref[t][np.isinf(ref[t])])
     fine = [t for t in range(T) if t not in (3, 7, 9, 11)]
     _check(torch.from_numpy(y[fine]), x[fine], w.astype(np.float64))
+
+
+@pytest.mark.parametrize("gtype", [8, 12, 13, 14])
+@pytest.mark.parametrize("T", [9, 70, 130])
+def test_weights_whole(gtype, T):
+    """Weights enter with all their fp32 bits. Rows hold a block at the scales 1707, 1706 and 1 x 2^-10
+    (the last with codes of its own) against tokens +-1 with the signs +, -, -, so the sums cancel to
+    2^-10 of their products. All products are multiples of 2^-10 whose absolute sum stays under 2^14:
+    fp32 adds them exactly in any order, and every result is the exact sum's nearest bf16."""
+    rng = np.random.default_rng(gtype + T)
+    N, (be, ts), dof = 64, ops.gguf_block_info(gtype), 208 if gtype == 14 else 0
+    base = synth.make_gguf(rng, gtype, 2 * N * be).reshape(2, N, ts)
+    if gtype == 14:
+        base[:, :, 192:208] = rng.integers(-15, 16, (2, N, 16)).astype(np.int8).view(np.uint8)
+    blocks = np.stack([base[0], base[0], base[1]], 1)  # [N, 3, ts]
+    for i, d in enumerate((1707, 1706, 1)):
+        blocks[:, i, dof:dof + 2] = np.array([d * 2.0 ** -10], np.float16).view(np.uint8)
+        if gtype in (12, 13):
+            blocks[:, i, 2:4] = blocks[:, i, 0:2]  # dmin
+    w = og.dequant_tensor(blocks.reshape(-1), gtype, (N, 3 * be)).astype(np.float64)
+    x = np.zeros((T, 3, be))
+    for k in rng.permutation(be):
+        s = rng.choice([-1.0, 1.0], T)
+        x[:, 0, k], x[:, 1, k], x[:, 2, k] = s, -s, -s
+        if (np.abs(x[0]).reshape(-1) @ np.abs(w).T).max() >= 2.0 ** 14:
+            x[:, :, k] = 0.0
+            break
+    x = x.reshape(T, -1)
+    assert (w * 2 ** 10 == np.round(w * 2 ** 10)).all() and np.count_nonzero(x[0]) >= 6
+    y = ops.gguf_matvec(torch.from_numpy(x).to(torch.bfloat16).cuda(), dev_u8(blocks.reshape(-1)), gtype, N, 3 * be)
+    ref = torch.from_numpy((x @ w.T).astype(np.float32)).to(torch.bfloat16)
+    assert torch.equal(y.cpu(), ref)

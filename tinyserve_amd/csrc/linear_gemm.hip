@@ -14,13 +14,13 @@
 // buffer-to-LDS copies into one of two XOR-swizzled tiles. The KW partial sums meet in LDS.
 //
 // Precision. bf16 x MXFP4 and bf16 x bf16 products are exact in the bf16 MFMA. A GGUF weight is
-// the fp32 value the block format defines (decode_unit's), carried as two bf16 terms, hi = its
-// upper 16 bits and lo = bf16(w - hi): 2^-17 of the weight, where a bf16 result keeps 2^-9.
-// Measured against 64-bit sums (bf16 results, 9 .. 1536 tokens) the error is that of the fp32
-// row kernels, 1.7e-3 relative, all of it the rounding of y. Results with other output types
-// stay on those kernels. A sum that is not finite is formed again value by value in fp32
-// (lg_exact): an infinite activation or scale meets a zero lo term as NaN, where the plain
-// product may be infinite.
+// the fp32 value the block format defines (decode_unit's), carried whole as three bf16 terms of 8
+// significant bits each (lg_split), so its products are exact too and the sums are fp32, as in the
+// row kernels. (Two terms, the second rounded, keep 2^-16 of the weight, and sums that cancel come
+// out of the wrong bits. The third costs Q6_K 2048 x 4096, 24 tokens, 15.2 -> 18.0 us, Q4_K 4096 x
+// 2048, 512 tokens, 24.7 -> 30.2 us.) Results with other output types stay on the row kernels. A
+// sum that is not finite is formed again value by value in fp32 (lg_exact): an infinite activation
+// meets a zero term as NaN, where the plain product may be infinite.
 #include "fused_common.h"
 #include "mfma_tile.h"
 
@@ -155,21 +155,31 @@ __device__ __forceinline__ void lg_load(const LgParams& p, const LgBufs& b, uint
     }
 }
 
-// 16 values as packed bf16 words: hi = their upper halves, lo = the rest rounded to bf16.
-__device__ __forceinline__ void lg_split(const float (&v)[16], uint32_t (&hi)[8], uint32_t (&lo)[8]) {
+// Two bf16 words in one: the upper halves of a and b.
+__device__ __forceinline__ uint32_t lg_upper(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+// 16 values as three terms of packed bf16 words, upper half by upper half: each takes the 8 leading
+// significant bits of what the one before leaves, 24 in all, so v = t[0] + t[1] + t[2] exactly
+// (down to bf16's smallest number).
+__device__ __forceinline__ void lg_split(const float (&v)[16], uint32_t (&t)[3][8]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const uint32_t a = __float_as_uint(v[2 * i]), b = __float_as_uint(v[2 * i + 1]);
-        hi[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-        lo[i] = pack_bf16x2(v[2 * i] - __uint_as_float(a & 0xFFFF0000u), v[2 * i + 1] - __uint_as_float(b & 0xFFFF0000u));
+        float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+            t[k][i] = lg_upper(ua, ub);
+            a -= __uint_as_float(ua & 0xFFFF0000u), b -= __uint_as_float(ub & 0xFFFF0000u);
+        }
     }
 }
 
-// Unit i (0 .. 3) of the step as A operands: hi[4 s ..], lo[4 s ..] for K step s (lo only for
-// GGUF weights). H: the half super-block of an aligned K-quant row.
+// Unit i (0 .. 3) of the step as A operands: the terms' words 4 s .. 4 s + 3 for K step s (one term
+// unless the weights are GGUF). H: the half super-block of an aligned K-quant row.
+template <int F> constexpr int lg_terms() { return F == LG_MXFP4 || F == LG_BF16 ? 1 : 3; }
 template <int F, bool SD, int H>
 __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)[lg_nraw<F, SD>()], uint32_t row, int j,
-                                          int i, int g, uint32_t (&hi)[8], uint32_t (&lo)[8]) {
+                                          int i, int g, uint32_t (&t)[lg_terms<F>()][8]) {
     if constexpr (F == LG_MXFP4) {
         const uint32_t ob = (p.s_mis + row * (uint32_t)p.KU + (uint32_t)j) & 3u;
         const float s = e8m0_to_f32((__builtin_amdgcn_alignbyte(R[9], R[8], ob) >> (8 * i)) & 0xFFu);
@@ -177,11 +187,11 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
         for (int k = 0; k < 2; ++k) {
             const u32x4 v = __builtin_bit_cast(u32x4, expand(R[2 * i + k], s));
 #pragma unroll
-            for (int d = 0; d < 4; ++d) hi[4 * k + d] = v[d];
+            for (int d = 0; d < 4; ++d) t[0][4 * k + d] = v[d];
         }
     } else if constexpr (F == LG_BF16) {
 #pragma unroll
-        for (int d = 0; d < 8; ++d) hi[d] = R[8 * i + d];
+        for (int d = 0; d < 8; ++d) t[0][d] = R[8 * i + d];
     } else {
         float v[16];
         const uint32_t U = row * (uint32_t)p.KU + (uint32_t)(j + i);
@@ -219,7 +229,7 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
                 for (int e = 0; e < 4; ++e) v[4 * w + e] = a * (float)((q >> (8 * e)) & 0xFFu) - c;
             }
         } else {
-            const uint32_t u = SD ? U & 7u : (uint32_t)(4 * H + i), t = u & 3u;
+            const uint32_t u = SD ? U & 7u : (uint32_t)(4 * H + i), um = u & 3u;
             const uint32_t o = p.w_mis + 210u * (U >> 3), ob = o & 3u;  // 0 or 2
             uint32_t ql[4], qh[4];
             float d, dd;
@@ -236,7 +246,7 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
                 d = f16_bits_to_f32(R[18] >> (8 * ob));
                 dd = 0.25f * (d * (float)(int8_t)(sw & 0xFFu));
             }
-            const uint32_t shl = 4 * (t >> 1), shh = 2 * t;
+            const uint32_t shl = 4 * (um >> 1), shh = 2 * um;
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 // four signed bytes 4 (q - 32): q ^ 32 is q - 32 in 6-bit two's complement
@@ -246,7 +256,7 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
                 for (int e = 0; e < 4; ++e) v[4 * w + e] = dd * (float)(int8_t)((q >> (8 * e)) & 0xFFu);
             }
         }
-        lg_split(v, hi, lo);
+        lg_split(v, t);
     }
 }
 
@@ -291,7 +301,7 @@ template <int F, int MT, int KW, bool SD>
 __global__ void __launch_bounds__(LG_THREADS) lin_gemm_kernel(LgParams p) {
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int RW = 8 / KW, ROWS = 32 * RW, TOK = 32 * MT, STEP = 128 * KW, CH = STEP / 8, XB = lg_xbytes(MT, KW);
-    constexpr int NX = MT * KW, NR = lg_nraw<F, SD>(), TERMS = F == LG_MXFP4 || F == LG_BF16 ? 1 : 2;
+    constexpr int NX = MT * KW, NR = lg_nraw<F, SD>(), TERMS = lg_terms<F>();
     // Workgroups are dealt round the 8 XCDs by linear id: renumbered so that each XCD takes a
     // run of row tiles with all their token tiles (the weights of a row tile share one L2).
     const int tt = (p.T + TOK - 1) / TOK, total = (int)gridDim.x, lin = (int)blockIdx.x;
@@ -340,21 +350,20 @@ __global__ void __launch_bounds__(LG_THREADS) lin_gemm_kernel(LgParams p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (j + i >= p.KU) break;  // wave-uniform: past the row's end
-            uint32_t hi[8], lo[8];
-            lg_decode<F, SD, H>(p, R, row, j, i, g, hi, lo);
+            uint32_t w[TERMS][8];
+            lg_decode<F, SD, H>(p, R, row, j, i, g, w);
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const bf16x8 A = __builtin_bit_cast(bf16x8, u32x4{hi[4 * s], hi[4 * s + 1], hi[4 * s + 2], hi[4 * s + 3]});
                 const int c = (4 * (4 * kw + i) + 2 * g + s) ^ rr;
                 bf16x8 B[MT];
 #pragma unroll
                 for (int t = 0; t < MT; ++t) B[t] = *reinterpret_cast<const bf16x8*>(xr + t * (512 * CH) + 16 * c);
 #pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B[t], acc[t], 0, 0, 0);
-                if constexpr (TERMS == 2) {
-                    const bf16x8 Al = __builtin_bit_cast(bf16x8, u32x4{lo[4 * s], lo[4 * s + 1], lo[4 * s + 2], lo[4 * s + 3]});
+                for (int m = 0; m < TERMS; ++m) {
+                    const bf16x8 A =
+                        __builtin_bit_cast(bf16x8, u32x4{w[m][4 * s], w[m][4 * s + 1], w[m][4 * s + 2], w[m][4 * s + 3]});
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(Al, B[t], acc[t], 0, 0, 0);
+                    for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B[t], acc[t], 0, 0, 0);
                 }
             }
         }
