@@ -113,6 +113,36 @@ def test_not_finite(fmt):
     _check(torch.from_numpy(y[fine]), x[fine], w.astype(np.float64))
 
 
+def _us(fn, n=20):
+    best = float("inf")
+    for _ in range(4):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(n):
+            fn()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+def test_not_finite_cost():
+    """One NaN token must not hold up the call: its results are NaN after one look at the token (a
+    thread forming 8 results one after the other in fp32 took 60 times the call's time)."""
+    rng = np.random.default_rng(3)
+    N, K, T = 2048, 4096, 24
+    w = dev_u8(synth.make_gguf(rng, 14, N * K))
+    _, x = _x(rng, T, K)
+    y = ops.gguf_matvec(x, w, 14, N, K)
+    t0 = _us(lambda: ops.gguf_matvec(x, w, 14, N, K))
+    x[5, 17] = float("nan")
+    z = ops.gguf_matvec(x, w, 14, N, K)
+    t1 = _us(lambda: ops.gguf_matvec(x, w, 14, N, K))
+    rest = [t for t in range(T) if t != 5]
+    assert z[5].isnan().all() and torch.equal(z[rest], y[rest])
+    assert t1 < 4 * t0, f"{t0:.1f} us, with a NaN token {t1:.1f}"
+
+
 @pytest.mark.parametrize("gtype", [8, 12, 13, 14])
 @pytest.mark.parametrize("T", [9, 70, 130])
 def test_weights_whole(gtype, T):

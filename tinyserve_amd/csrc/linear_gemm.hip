@@ -260,35 +260,82 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
     }
 }
 
-// The dot product of weight row n and token t in fp32, value by value (for results that the
-// operands leave not finite). MXFP4: per block the codes' dot product, then its scale.
+// Unit j's part of the dot product of weight row n and token t in fp32, value by value (MXFP4: the
+// codes' dot product, then the block's scale).
 template <int F>
-__device__ float lg_exact(const LgParams& p, int t, int n) {
-    const uint16_t* xr = p.x + (int64_t)t * p.K;
-    float s = 0.0f;
-    for (int j = 0; j < p.KU; ++j) {
-        const int64_t U = (int64_t)n * p.KU + j;
-        float v[32], d = 0.0f;
-        if constexpr (F == LG_MXFP4) {
+__device__ __forceinline__ float lg_exact(const LgParams& p, int t, int n, int j) {
+    const int64_t U = (int64_t)n * p.KU + j;
+    const u32x4* xr = reinterpret_cast<const u32x4*>(p.x + (int64_t)t * p.K + 32 * j);
+    float v[32], d = 0.0f;
+    if constexpr (F == LG_MXFP4) {
+        const u32x4 c = reinterpret_cast<const u32x4*>(p.w)[U];
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const uint32_t c = p.w[16 * U + k];
-                v[2 * k] = e2m1_to_f32(c & 15u);
-                v[2 * k + 1] = e2m1_to_f32(c >> 4);
-            }
-        } else if constexpr (F == LG_BF16) {
+        for (int k = 0; k < 32; ++k) v[k] = e2m1_to_f32((c[k >> 3] >> (4 * (k & 7))) & 15u);
+    } else if constexpr (F == LG_BF16) {
 #pragma unroll
-            for (int k = 0; k < 32; ++k) v[k] = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(p.w)[32 * U + k]);
-        } else {
-            using Tr = GgufTraits<F>;
-            decode_unit<F, Tr::FAST_A>(p.w + p.w_mis + U / Tr::UPB * Tr::TS, (int)(U % Tr::UPB), v);
+        for (int i = 0; i < 4; ++i) {
+            const u32x4 c = reinterpret_cast<const u32x4*>(p.w)[4 * U + i];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[8 * i + k] = __uint_as_float(k & 1 ? c[k >> 1] & 0xFFFF0000u : c[k >> 1] << 16);
         }
-#pragma unroll
-        for (int k = 0; k < 32; ++k) d = fmaf(v[k], bf16_bits_to_f32(xr[32 * j + k]), d);
-        if constexpr (F == LG_MXFP4) d *= e8m0_to_f32(p.scales[p.s_mis + U]);
-        s += d;
+    } else {
+        using Tr = GgufTraits<F>;
+        decode_unit<F, Tr::FAST_A>(p.w + p.w_mis + U / Tr::UPB * Tr::TS, (int)(U % Tr::UPB), v);
     }
-    return s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const u32x4 x = xr[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d = fmaf(v[8 * i + k], __uint_as_float(k & 1 ? x[k >> 1] & 0xFFFF0000u : x[k >> 1] << 16), d);
+    }
+    if constexpr (F == LG_MXFP4) d *= e8m0_to_f32(p.scales[p.s_mis + U]);
+    return d;
+}
+
+__device__ __forceinline__ bool lg_finite(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
+
+// The results of a wave (lane: rows n .. n + 7 of token t, `live` of them) that are not finite, again
+// in fp32: NaN for all of a token that holds one, else the whole wave forms one after the other, its
+// lanes over the units. us per call, finite / one token with a NaN / one with an infinity / all
+// tokens with a NaN / with an infinity: Q6_K 2048 x 4096, 24 tokens 18 / 20 / 76 / 47 / 945, Q4_K 4096 x
+// 2048, 512 tokens 32 / 35 / 143 / 47 / 1160, MXFP4 5760 x 2880, 77 tokens 13 / 15 / 256 / 27 / 2230 (a
+// thread for 8 results, one after the other: 950, 365, 2200 for the one NaN; the row kernels take
+// 59, 1210, 247 for any values).
+template <int F>
+__device__ __forceinline__ void lg_redo(const LgParams& p, int t, int n, int live, float (&v)[8]) {
+    const int lane = threadIdx.x & 63;
+    uint32_t bad = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bad |= e < live && !lg_finite(v[e]) ? 1u << e : 0u;
+    for (uint64_t m = __ballot(bad != 0), fine = 0; m;) {  // fine: lanes whose token is known to hold no NaN
+        const int l = __ffsll((unsigned long long)m) - 1, tl = __builtin_amdgcn_readlane(t, l);
+        if (!(fine >> l & 1)) {
+            bool nan = false;
+            for (int c = lane; c < p.K / 8; c += 64) {
+                const u32x4 x = *reinterpret_cast<const u32x4*>(p.x + (int64_t)tl * p.K + 8 * c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) nan |= (x[i] & 0x7FFFu) > 0x7F80u || (x[i] & 0x7FFF0000u) > 0x7F800000u;
+            }
+            const uint64_t same = __ballot(t == tl);
+            if (__ballot(nan)) {
+#pragma unroll
+                for (int d = 0; d < 8; ++d) v[d] = t == tl && (bad >> d & 1) ? __uint_as_float(0x7FC00000u) : v[d];
+                m &= ~same;
+                continue;
+            }
+            fine = same;
+        }
+        const int nl = __builtin_amdgcn_readlane(n, l);
+        for (uint32_t w = __builtin_amdgcn_readlane(bad, l); w; w &= w - 1) {
+            const int e = __builtin_ctz(w);
+            float s = 0.0f;
+            for (int j = lane; j < p.KU; j += 64) s += lg_exact<F>(p, tl, nl + e, j);
+            s = wave_sum(s);
+#pragma unroll
+            for (int d = 0; d < 8; ++d) v[d] = lane == l && d == e ? s : v[d];
+        }
+        m &= m - 1;
+    }
 }
 
 __host__ __device__ constexpr int lg_xbytes(int MT, int KW) { return 32 * MT * 256 * KW; }  // one token tile of a step
@@ -406,9 +453,9 @@ __global__ void __launch_bounds__(LG_THREADS) lin_gemm_kernel(LgParams p) {
             *reinterpret_cast<float4*>(stage + (kw * TOK + 32 * t + rr) * SS + 32 * rg + 8 * u + 4 * g) =
                 make_float4(acc[t][4 * u], acc[t][4 * u + 1], acc[t][4 * u + 2], acc[t][4 * u + 3]);
     __syncthreads();
+    static_assert(TOK * (ROWS / 8) % 64 == 0, "whole waves below");
     for (int i = tid; i < TOK * (ROWS / 8); i += LG_THREADS) {
         const int tk = i / (ROWS / 8), c = 8 * (i % (ROWS / 8)), t = t0 + tk, n = n0 + c;
-        if (t >= p.T || n >= p.N) continue;
         float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < KW; ++k) {
@@ -417,30 +464,29 @@ __global__ void __launch_bounds__(LG_THREADS) lin_gemm_kernel(LgParams p) {
             v[0] += a.x, v[1] += a.y, v[2] += a.z, v[3] += a.w;
             v[4] += d.x, v[5] += d.y, v[6] += d.z, v[7] += d.w;
         }
-        const int live = p.N - n < 8 ? p.N - n : 8;
-        bool fin = true;
+        const int live = t < p.T ? (p.N - n < 8 ? p.N - n : 8) : 0;  // 0 or less: none
+        float b[8];  // without a bias -0, which leaves every sum as it is
 #pragma unroll
-        for (int e = 0; e < 8; ++e) fin = fin && (__float_as_uint(v[e]) & 0x7F800000u) != 0x7F800000u;
-        if (!fin) {
-            for (int e = 0; e < live; ++e) {  // rolled: one copy of the fp32 loop
-                const float s = lg_exact<F>(p, t, n + e);
-#pragma unroll
-                for (int d = 0; d < 8; ++d) v[d] = d == e && (__float_as_uint(v[d]) & 0x7F800000u) == 0x7F800000u ? s : v[d];
-            }
-        }
+        for (int e = 0; e < 8; ++e) b[e] = -0.0f;
         if (p.bias) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (e < live) v[e] += load_act(p.bias, p.bias_dtype, n + e);
+                if (e < live) b[e] = load_act(p.bias, p.bias_dtype, n + e);
         }
+        uint32_t top = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) top = max(top, __float_as_uint(v[e]) << 1);
+        if (__builtin_expect(__ballot(live > 0 && top >= 0xFF000000u) != 0, 0)) lg_redo<F>(p, t, n, live, v);
+        uint32_t o[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) o[d] = pack_bf16x2(v[2 * d] + b[2 * d], v[2 * d + 1] + b[2 * d + 1]);
         uint16_t* dst = p.y + (int64_t)t * p.N + n;
         if (p.y_vec) {
-            *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
-                                                        pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+            if (live > 0) *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (e < live) dst[e] = f32_to_bf16_bits(v[e]);
+                if (e < live) dst[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1)));
         }
     }
 }
