@@ -143,6 +143,21 @@ def test_not_finite_cost():
     assert t1 < 4 * t0, f"{t0:.1f} us, with a NaN token {t1:.1f}"
 
 
+@pytest.mark.parametrize("gtype", [8, 12, 14])
+@pytest.mark.parametrize("N,T", [(64, 16), (32, 33)])
+def test_few_rows_long_k(gtype, N, T):
+    """Few rows of a long K, where the GEMM has one or two workgroups, take the row kernel, as fp32
+    tokens do (the GEMM took 2.5 to 5 times as long)."""
+    rng = np.random.default_rng(gtype + N)
+    K = 16384
+    data = synth.make_gguf(rng, gtype, N * K)
+    x, xd = _x(rng, T, K)
+    w, xf = dev_u8(data), xd.float()
+    _check(ops.gguf_matvec(xd, w, gtype, N, K), x, og.dequant_tensor(data, gtype, (N, K)).astype(np.float64))
+    t0, t1 = _us(lambda: ops.gguf_matvec(xf, w, gtype, N, K)), _us(lambda: ops.gguf_matvec(xd, w, gtype, N, K))
+    assert t1 < 1.6 * t0, f"{t1:.1f} us, fp32 tokens {t0:.1f}"
+
+
 @pytest.mark.parametrize("gtype", [8, 12, 13, 14])
 @pytest.mark.parametrize("T", [9, 70, 130])
 def test_weights_whole(gtype, T):

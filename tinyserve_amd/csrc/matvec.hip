@@ -278,14 +278,37 @@ using namespace tsa;
 
 // Up to this many tokens per call run on the super-block streaming matvec (gguf_matvec.hip,
 // one workgroup column per token). More bf16 tokens take the matrix cores (linear_gemm.hip;
-// Q4_K 4096 x 2048, 512 tokens: 1209 us on the row kernel above, 29 us there), other types and
-// alignments reuse each decoded unit across a chunk of tokens in the row kernel.
+// Q4_K 4096 x 2048, 512 tokens: 1209 us on the row kernel above, 32 us there) where that is the
+// faster; other types and alignments reuse each decoded unit across a chunk of tokens in the row
+// kernel.
 constexpr int64_t GQ_MATVEC_MAX_T = 8;
+// The row kernel against the linear GEMM where few rows meet a long K: one of the GEMM's workgroups
+// walks all of K, 1024 values at a time, however few there are. Both times in ns, fitted to 2092
+// measured cells (4 types, K 256 .. 16384, 32 .. 2048 rows, 9 .. 96 tokens), where the choice is
+// within 6% of the better one in all but 14 (1.21 x the worst); the GEMM alone is not in 676. us, row
+// kernel / GEMM: Q8_0 64 x 16384, 16 tokens 12.9 / 64.6, 128 x 2048, 16 tokens 9.0 / 11.6, 1024 x 2048,
+// 16 tokens 13.0 / 11.9; Q6_K 128 x 2880, 16 tokens 12.1 / 20.2; Q4_K 128 x 4096, 16 tokens 15.4 / 13.6.
+static bool gguf_gemm_better(int type, int64_t T, int64_t N, int64_t K) {
+    const bool sd = type != 8 && K % 256 != 0;  // K-quant rows that start inside a super-block
+    if (K <= 512 || (K <= 1024 && type != 8 && !(sd && type == 14))) return true;
+    const int64_t step = type == 8 ? 3700 : type == 12 ? (sd ? 3300 : 2700) : type == 13 ? (sd ? 3500 : 2850) : (sd ? 5650 : 3750);
+    const int64_t gemm = 2500 + (K + 1023) / 1024 * step;
+    const int tch = pick_tch(T, K);
+    const int64_t rounds = ((N + ROWS_PER_WG - 1) / ROWS_PER_WG * ((T + tch - 1) / tch) + 255) / 256;
+    const int64_t one = K <= 1024 ? 7500 : K <= 2048 ? 9000 : K <= 4096 && (type == 12 || type == 13) ? 14500 : 12000;
+    const int64_t row = 5000 + 550 * rounds * tch * K / 1024;
+    return gemm <= (row > one ? row : one);
+}
 // MXFP4: the linear GEMM (linear_gemm.hip) above 32 tokens, and from 9 on where the matvec's
 // grid, one workgroup per 16 rows and 8 tokens, passes 512: 5760 x 2880 at 9 / 24 / 32 tokens
 // takes 8.2 / 8.1 / 8.2 us there and 9.6 / 19.2 / 22.6 here, 1536 x 2048 at 9 / 24 (192 / 288
-// workgroups) 7.0 / 7.2 against 5.4 / 7.2, 2048 x 768 at 32 (512) 5.5 against 4.7.
-static bool mx_gemm_better(int64_t T, int64_t N) { return T > 32 || (T > 8 && (N + 15) / 16 * ((T + 7) / 8) > 512); }
+// workgroups) 7.0 / 7.2 against 5.4 / 7.2, 2048 x 768 at 32 (512) 5.5 against 4.7. A few rows of a
+// long K stay on the row kernel (us there / on the GEMM: 64 x 8192, 64 tokens 13.2 / 17.1, 96 x 8192, 48
+// tokens 20.5 / 17.1, 32 x 16384, 48 tokens 13.4 / 30.2; 64 x 4096, 64 tokens 10.9 / 10.3).
+static bool mx_gemm_better(int64_t T, int64_t N, int64_t K) {
+    if (T > 32) return K <= 4096 || N * T > 4096;
+    return T > 8 && (N + 15) / 16 * ((T + 7) / 8) > 512;
+}
 
 extern "C" int tsa_gguf_matvec(int ggml_type, const void* w, int64_t w_bytes, const void* x, int x_dtype, int64_t T,
                                int64_t K, void* y, int y_dtype, int64_t N, void* stream) {
@@ -316,7 +339,8 @@ extern "C" int tsa_gguf_matvec(int ggml_type, const void* w, int64_t w_bytes, co
         return gs_matvec(ggml_type, wb, w_bytes, x, x_dtype, T, K, y, y_dtype, N, st);
     if (T <= GQ_MATVEC_MAX_T && !*gq_matvec_unsupported(ggml_type, w, T, K, N, x_dtype))
         return gq_matvec(ggml_type, wb, w_bytes, x, x_dtype, T, K, y, y_dtype, N, st);
-    if (T > GQ_MATVEC_MAX_T && lg_gguf_supported(ggml_type, w, x, x_dtype, y_dtype, T, N, K))
+    if (T > GQ_MATVEC_MAX_T && lg_gguf_supported(ggml_type, w, x, x_dtype, y_dtype, T, N, K) &&
+        gguf_gemm_better(ggml_type, T, N, K))
         return lg_gguf(ggml_type, wb, w_bytes, x, T, K, y, N, st);
     const bool a16 = (reinterpret_cast<uintptr_t>(w) & 15) == 0, a2 = (reinterpret_cast<uintptr_t>(w) & 1) == 0;
     const int tch = pick_tch(T, K);
@@ -350,7 +374,7 @@ extern "C" int tsa_mxfp4_matvec(const void* blocks, const void* scales, const vo
     const uint8_t* bl = static_cast<const uint8_t*>(blocks);
     const uint8_t* sc = static_cast<const uint8_t*>(scales);
     hipStream_t st = as_stream(stream);
-    if (mx_gemm_better(T, N) && lg_mxfp4_supported(blocks, x, x_dtype, y_dtype, T, N, K))
+    if (mx_gemm_better(T, N, K) && lg_mxfp4_supported(blocks, x, x_dtype, y_dtype, T, N, K))
         return lg_mxfp4(bl, sc, bias, bias_dtype, x, T, y, N, K, st);
     // bf16 tokens, a few at a time: the matrix-core form (mx_matvec.hip)
     if (T <= 32 && mxm_supported(blocks, x, x_dtype, N, K))

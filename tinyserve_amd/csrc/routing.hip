@@ -275,7 +275,6 @@ int lg_bf16(const void* w, const void* bias, int bias_dtype, const void* x, int6
 
 using namespace tsa;
 
-
 extern "C" int tsa_router_logits(const void* x, int x_dtype, int64_t T, int64_t H, const void* w, int w_dtype,
                                  const void* bias, int bias_dtype, int64_t E, void* out, int out_dtype, void* stream) {
     clear_error();
@@ -305,8 +304,9 @@ extern "C" int tsa_router_logits(const void* x, int x_dtype, int64_t T, int64_t 
         return TSA_OK;
     }
     // bf16 batches on the matrix cores (linear_gemm.hip; 128 experts x 2048, 2048 tokens: 101 us on
-    // router_logits_kernel, 9.4 us there; 5 tokens: 10.9 and 8.1 us)
-    if (lg_bf16_supported(w, w_dtype, x, x_dtype, out_dtype, T, E, H))
+    // router_logits_kernel, 9.1 us there; 5 tokens: 10.9 and 8.1 us), but not a few tokens of a short H
+    // (128 x 512, 5 / 7 / 8 tokens: 4.6 / 5.3 / 5.6 us here, 5.7 there; 128 x 768, 5 tokens 6.7 and 5.7)
+    if ((T >= 8 || H > 512) && lg_bf16_supported(w, w_dtype, x, x_dtype, out_dtype, T, E, H))
         return lg_bf16(w, bias, bias_dtype, x, T, out, E, H, as_stream(stream));
     hipLaunchKernelGGL(router_logits_kernel, dim3((unsigned)((E + 3) / 4), (unsigned)((T + RT - 1) / RT)), dim3(256), 0,
                        as_stream(stream), x, x_dtype, T, (int)H, w, w_dtype, bias, bias_dtype, (int)E, out, out_dtype);
