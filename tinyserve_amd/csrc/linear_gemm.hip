@@ -504,15 +504,20 @@ hipError_t lg_launch(const LgParams& p, hipStream_t st) {
 }
 
 // The tile (32 MT tokens x 256 / KW rows): the one with the least rounds x round time, a round
-// being one workgroup on every CU. A round's relative times are measured (Q4_K, K 2048, one
-// round of each: 35 / 25 / 15 / 12.3 / 8.1 us; Q6_K and Q8_0 keep the order). More K groups per
-// workgroup shorten a round and re-read the tokens more often, more tokens per workgroup share
-// a decoded weight. Q4_K 4096 x 2048, tokens: picked tile and its time, the next best's:
-// 24: 1x8 8.2 / 12.3, 130: 2x4 16.1 / 20.4, 512: 2x2 29.4 / 32.6, 1536: 4x2 85.6 / 101 us.
+// being one workgroup on every CU. More K groups per workgroup shorten a round and re-read the
+// tokens more often, more tokens per workgroup share a decoded weight. A round of each, us, at K
+// 2048 / 8192: Q4_K 9.1 13.9 18.4 32.3 48.2 / 30.1 48.5 62.6 113.8 178.8, Q8_0 12.6 20.5 25.3 39.6
+// 55.2 / 40.3 65.2 79.5 144.7 208.7, Q6_K 11.1 17.9 22.0 38.2 53.6 / 36.2 62.4 74.8 140.6 196.8, bf16 9.0
+// 15.3 17.9 29.3 37.5 / 28.0 47.9 55.3 131.2 150.5, MXFP4 7.2 9.3 11.6 20.2 29.6 / 19.8 31.4 37.4 61.4
+// 87.5. With the costs here the pick is the fastest of the five in all of 230 calls measured with
+// each tile (GGUF N 512 .. 5760, K 2048 .. 8192, 20 .. 1500 tokens; bf16 128 and 512 rows). MXFP4 has
+// its own: two of its 2x2 workgroups share a CU (registers and LDS), so 4x2 costs more against
+// them (5760 x 2880, 1024 tokens: 49 and 63 us); within 3% of the fastest in all of 70 calls.
 template <int F, bool SD>
 hipError_t lg_pick(const LgParams& p, hipStream_t st) {
     struct Tile { int mt, kw, cost; };
-    constexpr Tile tiles[5] = {{1, 8, 81}, {1, 4, 123}, {2, 4, 150}, {2, 2, 250}, {4, 2, 350}};
+    constexpr bool MX = F == LG_MXFP4;
+    constexpr Tile tiles[5] = {{1, 8, 81}, {1, 4, MX ? 105 : 123}, {2, 4, MX ? 130 : 150}, {2, 2, MX ? 211 : 250}, {4, 2, MX ? 356 : 350}};
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
     int best = 0;
     int64_t least = INT64_MAX;
