@@ -216,10 +216,10 @@ def test_gguf_grouped_prefill_straddling_rows(types, H, I, pad):
 
 
 @pytest.mark.parametrize("types,H,I,pad", [((12, 12, 12), 64, 32, 0), ((14, 14, 14), 96, 32, 6), ((13, 13, 14), 800, 384, 0),
-                                           ((12, 12, 14), 512, 256, 0)])
+                                           ((12, 12, 14), 512, 256, 0), ((8, 8, 8), 512, 256, 0), ((8, 8, 8), 800, 352, 6)])
 def test_gguf_grouped_prefill_tile_edges(types, H, I, pad):
     """Aligned rows, and straddling rows of 1, 2, 3, 12 and 25 units (a row inside one super-block, or over up to
-    five), weight rows that leave a tile part empty, and experts with 1, 32, 33, 64 and 65
+    five), Q8_0 with a whole and a partial last piece, weight rows that leave a tile part empty, and experts with 1, 32, 33, 64 and 65
     sorted rows (one or two blocks of 32, a second tile)."""
     rng = np.random.default_rng(500 + H + I + pad)
     loads = [1, 32, 33, 64, 65]

@@ -3,6 +3,9 @@ tsa_router_logits for many bf16 tokens: tile edges, ragged sizes, every tile sha
 start inside a super-block, unaligned weights and results that are not finite."""
 from __future__ import annotations
 
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -45,6 +48,45 @@ def test_gguf_linear(gtype, N, K, T):
         pytest.skip("not a whole number of super-blocks")
     x, xd = _x(rng, T, K)
     _check(ops.gguf_matvec(xd, dev_u8(data), gtype, N, K), x, og.dequant_tensor(data, gtype, (N, K)).astype(np.float64))
+
+
+def _tile(N, T, mxfp4):
+    """The tile lg_pick takes (32 x first tokens, 256 / second rows), from the source's table."""
+    src = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tinyserve_amd", "csrc",
+                            "linear_gemm.hip")).read()
+    table = re.findall(r"\{(\d), (\d), (?:MX \? (\d+) : )?(\d+)\}", re.search(r"constexpr Tile tiles\[5\] = (.*);", src)[1])
+    assert len(table) == 5
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+
+    def cost(mt, kw, mx, other):
+        wgs = -(-N // (256 // int(kw))) * -(-T // (32 * int(mt)))
+        return -(-wgs // cus) * int(mx if mx and mxfp4 else other)
+
+    return min(((int(mt), int(kw)) for mt, kw, *_ in table), key={(int(t[0]), int(t[1])): cost(*t) for t in table}.get)
+
+
+@pytest.mark.parametrize("tile,T", [((1, 8), 20), ((1, 4), 95), ((2, 4), 130), ((2, 2), 499), ((4, 2), 1020)])
+@pytest.mark.parametrize("fmt,K", [(8, 1312), (12, 1280), (13, 1280), (14, 1280), (12, 1312), (13, 1312), (14, 1312),
+                                   ("mxfp4", 1312), ("bf16", 1312)])
+def test_tiles(fmt, K, tile, T):
+    """Each tile over several K steps (1024, 512 or 256 values each) with a partial last one wherever
+    the format allows it, in whole and straddling rows, with ragged rows and tokens."""
+    N = 4088
+    assert _tile(N, T, fmt == "mxfp4") == tile
+    rng = np.random.default_rng(K + T)
+    x, xd = _x(rng, T, K)
+    if fmt == "mxfp4":
+        blocks = rng.integers(0, 256, size=(N, K // 32, 16), dtype=np.uint8)
+        scales = rng.integers(110, 130, size=(N, K // 32), dtype=np.uint8)
+        w = omx.dequant_mxfp4_no_transpose(blocks, scales, "f32")
+        y = ops.mxfp4_matvec(xd, torch.from_numpy(blocks).cuda(), torch.from_numpy(scales).cuda())
+    elif fmt == "bf16":
+        wt = torch.from_numpy(rng.normal(0.0, K ** -0.5, (N, K)).astype(np.float32)).to(torch.bfloat16)
+        w, y = wt.float().numpy(), ops.router_logits(xd, wt.cuda())
+    else:
+        data = synth.make_gguf(rng, fmt, N * K)
+        w, y = og.dequant_tensor(data, fmt, (N, K)), ops.gguf_matvec(xd, dev_u8(data), fmt, N, K)
+    _check(y, x, w.astype(np.float64))
 
 
 @pytest.mark.parametrize("gtype,K", [(8, 96), (14, 512), (14, 288)])
