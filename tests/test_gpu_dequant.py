@@ -117,3 +117,28 @@ def test_mxfp4_dequant_unaligned_output(dtype, offset):
     out = buf[offset : offset + want.numel()]
     ops.mxfp4_dequant(blocks, scales, dtype=dtype, out=out)
     assert torch.equal(out.view_as(want), want) and not buf[:offset].any() and not buf[offset + want.numel() :].any()
+
+
+@pytest.mark.parametrize("fmt", [12, "mxfp4"])
+def test_dequant_more_than_one_launch(fmt):
+    """2^35 values: four threads a unit make 2^32 threads, more than one launch takes. Repeated
+    data, so the values around every launch's edges (2^33 apart) are those of one repeat."""
+    n, P = 1 << 35, 1 << 20
+    if torch.cuda.mem_get_info()[0] < 100 << 30:
+        pytest.skip("needs 100 GiB free")
+    rng = np.random.default_rng(35)
+    if fmt == "mxfp4":
+        blocks = torch.from_numpy(rng.integers(0, 256, (P // 4096, 128, 16), dtype=np.uint8)).cuda()
+        scales = torch.from_numpy(rng.integers(110, 130, (P // 4096, 128), dtype=np.uint8)).cuda()
+        ref = ops.mxfp4_dequant(blocks, scales).view(-1)
+        out = ops.mxfp4_dequant(blocks.repeat(n // P, 1, 1), scales.repeat(n // P, 1)).view(-1)
+    else:
+        data = dev_u8(synth.make_gguf(rng, fmt, P))
+        ref = ops.gguf_dequant(data, fmt, (P,), dtype=torch.bfloat16)
+        out = ops.gguf_dequant(data.repeat(n // P), fmt, (n,), dtype=torch.bfloat16)
+    ref = ref.view(torch.int16)
+    for e in range(0, n, 1 << 33):
+        for at in ({0, n - P} if e == 0 else {e - P, e}):
+            assert torch.equal(out[at:at + P].view(torch.int16), ref), at
+    del out
+    torch.cuda.empty_cache()

@@ -140,6 +140,10 @@ __global__ void __launch_bounds__(256) mxfp4_dequant_t_kernel(const uint8_t* __r
     }
 }
 
+// 32-value units per launch: a launch takes fewer than 2^32 threads, four per unit. A multiple of a
+// super-block's 8, and of 16 bytes in every type's blocks and output.
+constexpr int64_t LAUNCH_UNITS = (int64_t)1 << 28;
+
 inline unsigned grid_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
 }  // namespace
@@ -179,26 +183,31 @@ extern "C" int tsa_gguf_dequant(int ggml_type, const void* data, int64_t data_by
     const bool out_ok = (reinterpret_cast<uintptr_t>(out) & (out_dtype == TSA_F32 ? 15 : 3)) == 0;
     TSA_REQUIRE(out_ok, TSA_ERR_INVALID_ARG, "out must be %d-byte aligned", out_dtype == TSA_F32 ? 16 : 4);
     const int vec = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    const dim3 grid(grid_for(4 * n_units, 256)), block(256);
-    switch (ggml_type) {
-        case 8:
-            if (a2) hipLaunchKernelGGL((gguf_dequant_kernel<8, 2>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            else hipLaunchKernelGGL((gguf_dequant_kernel<8, 1>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            break;
-        case 12:
-            if (a16) hipLaunchKernelGGL((gguf_dequant_kernel<12, 16>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            else hipLaunchKernelGGL((gguf_dequant_kernel<12, 1>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            break;
-        case 13:
-            if (a16) hipLaunchKernelGGL((gguf_dequant_kernel<13, 16>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            else hipLaunchKernelGGL((gguf_dequant_kernel<13, 1>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            break;
-        default:
-            if (a2) hipLaunchKernelGGL((gguf_dequant_kernel<14, 2>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            else hipLaunchKernelGGL((gguf_dequant_kernel<14, 1>), grid, block, 0, st, d, n_units, out, out_dtype, vec);
-            break;
+    const dim3 block(256);
+    for (int64_t u0 = 0; u0 < n_units; u0 += LAUNCH_UNITS, d += LAUNCH_UNITS * 32 / be * ts) {
+        const int64_t nu = n_units - u0 < LAUNCH_UNITS ? n_units - u0 : LAUNCH_UNITS;
+        const dim3 grid(grid_for(4 * nu, 256));
+        void* o = static_cast<uint8_t*>(out) + u0 * 32 * dtype_size(out_dtype);
+        switch (ggml_type) {
+            case 8:
+                if (a2) hipLaunchKernelGGL((gguf_dequant_kernel<8, 2>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                else hipLaunchKernelGGL((gguf_dequant_kernel<8, 1>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                break;
+            case 12:
+                if (a16) hipLaunchKernelGGL((gguf_dequant_kernel<12, 16>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                else hipLaunchKernelGGL((gguf_dequant_kernel<12, 1>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                break;
+            case 13:
+                if (a16) hipLaunchKernelGGL((gguf_dequant_kernel<13, 16>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                else hipLaunchKernelGGL((gguf_dequant_kernel<13, 1>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                break;
+            default:
+                if (a2) hipLaunchKernelGGL((gguf_dequant_kernel<14, 2>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                else hipLaunchKernelGGL((gguf_dequant_kernel<14, 1>), grid, block, 0, st, d, nu, o, out_dtype, vec);
+                break;
+        }
+        TSA_LAUNCH_CHECK();
     }
-    TSA_LAUNCH_CHECK();
     return TSA_OK;
 }
 
@@ -216,8 +225,13 @@ extern "C" int tsa_mxfp4_dequant(const void* blocks, const void* scales, int64_t
         hipLaunchKernelGGL(mxfp4_dequant_t_kernel, dim3(grid_for(N * G, 256)), dim3(256), 0, as_stream(stream), bl, sc, N, G,
                            out, out_dtype);
     else
-        hipLaunchKernelGGL(mxfp4_dequant_kernel, dim3(grid_for(4 * N * G, 256)), dim3(256), 0, as_stream(stream), bl, sc, N * G,
-                           out, out_dtype, (int)((reinterpret_cast<uintptr_t>(out) & 15) == 0));
+        for (int64_t c0 = 0; c0 < N * G; c0 += LAUNCH_UNITS) {
+            const int64_t nc = N * G - c0 < LAUNCH_UNITS ? N * G - c0 : LAUNCH_UNITS;
+            hipLaunchKernelGGL(mxfp4_dequant_kernel, dim3(grid_for(4 * nc, 256)), dim3(256), 0, as_stream(stream), bl + 16 * c0,
+                               sc + c0, nc, static_cast<uint8_t*>(out) + c0 * 32 * dtype_size(out_dtype), out_dtype,
+                               (int)((reinterpret_cast<uintptr_t>(out) & 15) == 0));
+            TSA_LAUNCH_CHECK();
+        }
     TSA_LAUNCH_CHECK();
     return TSA_OK;
 }
