@@ -99,6 +99,17 @@ def test_wrappers_reject_host_tensors():
         ops.mxfp4_dequant(torch.zeros((1, 1, 16), dtype=torch.uint8), torch.zeros((1, 1), dtype=torch.uint8))
 
 
+def test_tensor_stream_with_and_without_the_raw_form(monkeypatch):
+    """The stream comes from torch's raw form where there is one, else from the public call."""
+    t = torch.zeros(1)
+    if _lib._raw_stream is not None:
+        monkeypatch.setattr(_lib, "_raw_stream", lambda dev: 100 + dev)
+        assert _lib.tensor_stream(t) == 100 + t.get_device()
+    monkeypatch.setattr(_lib, "_raw_stream", None)
+    monkeypatch.setattr(_lib, "stream_handle", lambda device: 7 if device == t.device else 0)
+    assert _lib.tensor_stream(t) == 7
+
+
 def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True,
                        text=True, timeout=300)

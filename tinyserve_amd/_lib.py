@@ -128,10 +128,14 @@ def stream_handle(device: torch.device | None = None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # not a public name
+
+
 def tensor_stream(t: torch.Tensor) -> int:
     """The current stream of a GPU tensor's device, as stream_handle gives it, without the
-    ``torch.cuda.Stream`` object around it (over 1 us of a 9 us call)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    ``torch.cuda.Stream`` object around it (over 1 us of a 9 us call) where this torch has the raw
+    form."""
+    return stream_handle(t.device) if _raw_stream is None else _raw_stream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
