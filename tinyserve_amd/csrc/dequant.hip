@@ -3,7 +3,7 @@
 // One thread decodes 8 consecutive values of a 32-value unit and writes them with 16-byte
 // stores, so a wave's stores are whole lines: what bounds the kernels is HBM (a unit per
 // thread, 64 bytes from its neighbour's, in dword stores took 78 us for 8192 x 4096 Q5_K to
-// bf16, 90 MB; this form 17.5 us, 5.1 TB/s). The four threads of a unit read its header again, from L1. The
+// bf16, 90 MB; this form 16.4 us, 5.5 TB/s). The four threads of a unit read its header again, from L1. The
 // arithmetic per value is formats.h's, to the bit.
 #include "formats.h"
 

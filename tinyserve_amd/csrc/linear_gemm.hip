@@ -223,7 +223,7 @@ __device__ __forceinline__ void lg_decode(const LgParams& p, const uint32_t (&R)
                 uint32_t q = (qs[w] >> sh) & 0x0F0F0F0Fu;
                 if constexpr (F == 13) q |= ((qh[w] >> u) & 0x01010101u) << 4;
                 // masked once for its four bytes (the compiler extracts each by itself otherwise:
-                // Q4_K 4096 x 2048, 512 tokens, 27.3 -> 24.4 us per call)
+                // Q4_K 4096 x 2048, 512 tokens, 27.3 -> 24.4 us per call, with two terms per weight)
                 asm("" : "+v"(q));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[4 * w + e] = a * (float)((q >> (8 * e)) & 0xFFu) - c;

@@ -332,7 +332,7 @@ extern "C" int tsa_gguf_matvec(int ggml_type, const void* w, int64_t w_bytes, co
     TSA_REQUIRE(w && x && y, TSA_ERR_INVALID_ARG, "null pointer");
     const uint8_t* wb = static_cast<const uint8_t*>(w);
     hipStream_t st = as_stream(stream);
-    // the sub-block stream (moe_decode_gs.hip) first, then the super-block matvec
+    // the sub-block stream (gguf_stream.hip) first, then the super-block matvec
     if (T <= GQ_MATVEC_MAX_T && !*gs_unsupported(ggml_type, K) && (reinterpret_cast<uintptr_t>(w) & 1) == 0 &&
         (reinterpret_cast<uintptr_t>(x) & 15) == 0 && N * K < ((int64_t)1 << 31) &&
         T * K * (x_dtype == TSA_F32 ? 4 : 2) < ((int64_t)1 << 32) - 16)

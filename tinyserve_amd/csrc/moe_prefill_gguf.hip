@@ -606,7 +606,8 @@ __global__ void __launch_bounds__(GF_THREADS, 2) gf_step_kernel(GfGemm p) {
 // (128 values each) that covers every ph. A lane reads its half of a super-block in 5 to 8
 // 16-byte loads, all at once and a super-block ahead: a row's cache lines are fetched once (16
 // bytes per step and wave took 2.4 times as long, the lines having left L1 in between). No
-// weight goes through LDS and its 64 KB leave room for two workgroups per CU.
+// weight goes through LDS and its 64 KB leave room for two workgroups per CU: at most 128 registers,
+// for which Q6_K spills 5 (gate_up) and 3 (down), reloaded in the K loop of two row blocks.
 // Bound by those row-divergent loads and the decode about equally (with one of them taken out
 // either gains 10 .. 15%, the matrix cores are a fifth busy). hidden = inter = 2880, 32 experts,
 // top 4, Q4_K gate / up and Q6_K down, gate_up + down in us, against pieces of 256 values staged

@@ -409,6 +409,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1) pf_gemm_kernel(PfGemm p) {
 //    only for its own kind: loads return in order, and a wave waiting for the activations 2
 //    pieces ahead would also wait for the weights 3 ahead;
 //  - a K step's operands are read while the step before multiplies, across the barrier;
+//  - the starts, ends and hand-overs of tiles keep about 155 scalar registers in lanes; a copy that
+//    reads one of them back has its wait states (TSA_COPY_WAIT);
 //  - stage positions are running byte offsets, LDS destinations immediates of the copies; the
 //    steady part of the loop has no tail checks, the tile's last 4 pieces are written out.
 // 2880 x 2880, top-4 of 32 experts, whole call (us; one loop with all reads and waits at its top
