@@ -101,7 +101,7 @@ def test_gguf_linear_2byte_aligned(gtype, K, offset):
 
 
 @pytest.mark.parametrize("N,K,T,offset", [(33, 32, 40, 0), (100, 96, 33, 1), (5760, 2880, 12, 0), (1536, 2080, 77, 2),
-                                          (2880, 160, 700, 3)])
+                                          (2880, 160, 700, 3), (64, 8192, 64, 0), (65, 8192, 64, 0), (33, 4128, 33, 2)])
 def test_mxfp4_linear(N, K, T, offset):
     rng = np.random.default_rng(N + K + T)
     blocks = rng.integers(0, 256, size=(N, K // 32, 16), dtype=np.uint8)
@@ -114,7 +114,8 @@ def test_mxfp4_linear(N, K, T, offset):
     _check(y, x, w, bias.astype(np.float64))
 
 
-@pytest.mark.parametrize("E,H,T", [(1, 32, 5), (60, 2048, 31), (33, 96, 200), (128, 2880, 700)])
+@pytest.mark.parametrize("E,H,T", [(1, 32, 5), (60, 2048, 31), (33, 96, 200), (128, 2880, 700), (128, 512, 7), (128, 512, 8),
+                                   (33, 544, 5)])
 def test_router_batch(E, H, T):
     rng = np.random.default_rng(E + H + T)
     x, xd = _x(rng, T, H)
